@@ -312,6 +312,14 @@ __device__ __forceinline__ float rowsum8(f16x8 v, float l) {
 }
 
 
+// Reference-rounding mode of a launch (the REFROUND template argument): 0 off, 1 the scores rounded as the
+// reference rounds them (score_value).
+template <int D, bool SOFTCAP, typename F>
+void with_ref_mode(bool ref, const AttnParams& p, F&& f) {
+  if (ref) f(std::integral_constant<int, 1>{});
+  else f(std::integral_constant<int, 0>{});
+}
+
 // Host-side validation of the attention arguments shared by the prefill, column and split-KV entry points
 // (nstrides strides, every third one a sequence stride), and the launch parameters they derive.
 int validate_attn(const char* op, const void* q, const void* k, int64_t B, int64_t Sq, int64_t Sk, int64_t Hq,
@@ -323,6 +331,10 @@ AttnParams make_params(const void* q, const void* k, const void* v, void* o, int
 // Software-pipelined head_dim-256 forward (attention_d256.hip) for 16-bit inputs without reference rounding:
 // 4 waves x 32 rows per workgroup (p.n_tiles counts 128-row query tiles).
 void launch_attn_d256_pipe(const AttnParams& p, bool bf16, hipStream_t st);
+
+// 16-bit forward (attention_fwd.h): picks the kernel and its tiling from the parameters (n_tiles is set there).
+void launch_attn_fwd_f16(const AttnParams& p, int D, bool ref, hipStream_t st);
+void launch_attn_fwd_bf16(const AttnParams& p, int D, bool ref, hipStream_t st);
 
 // fp32 inputs (attention_f32.hip): the forward and the column-score pass, rows per workgroup tile of both.
 int f32_rows_per_tile();
