@@ -11,14 +11,13 @@
 // Softmax runs in the exp2 domain with a lazily-updated row maximum: O and l are rescaled only when a row's
 // maximum grows by more than 2^8.
 //
-// Kernels. attn_fwd_dma_kernel (head_dim 128: 8 waves x 32 rows, 128-key tiles; head_dim 256: 4 waves, 64-key
-// tiles) copies K/V tiles global -> LDS with direct loads (global_load_lds_dwordx4) into a swizzled ring;
-// attn_fwd_kernel (head_dim 64) stages them through registers. Tiles a wave cannot see are skipped, and within
-// masked tiles dead 32-key blocks skip their MFMAs. attn_colsum_d128_kernel / attn_colsum_kernel recompute
-// P = exp2(s - lse) with one key per lane and sum (or test) it over the queries; attn_kf_rowlse_kernel is the
-// row pass of KeyFormer's perturbed softmax. Reference rounding (DGG_ATTN_REF_ROUNDING) rounds the scores as
-// the reference does on the GPU: matmul result to the input dtype, then the fp32 multiply by the reciprocal of
-// sqrt(D) (and of the soft-cap), rounded again.
+// Kernels. attn_fwd_dma_kernel (attention_fwd.h; 16-bit forward at every head_dim, except that head_dim 256 with fp32
+// scores runs on attention_d256.hip) copies K/V tiles global -> LDS with direct loads (global_load_lds_dwordx4) into a
+// swizzled ring. Tiles a wave cannot see are skipped, and within masked tiles dead 32-key blocks skip their MFMAs.
+// Here: attn_colsum_d128_kernel / attn_colsum_kernel recompute P = exp2(s - lse) with one key per lane and sum (or
+// test) it over the queries; attn_kf_rowlse_kernel is the row pass of KeyFormer's perturbed softmax. Reference rounding
+// (DGG_ATTN_REF_ROUNDING) rounds the scores as the reference does on the GPU: matmul result to the input dtype, then
+// the fp32 multiply by the reciprocal of sqrt(D) (and of the soft-cap), rounded again.
 // Workgroups are ordered longest-first and grouped by head inside each XCD so the K/V of a head stay in one L2.
 #include <algorithm>
 #include <cmath>
@@ -202,7 +201,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
       for (int j = 0; j < 16; ++j) l_run += fast_exp2(sacc[mb][j] - mu);
   };
 
-  // Tiles [t_full0, t_full1) need no mask for any row of the workgroup (as in attn_fwd_kernel).
+  // Tiles [t_full0, t_full1) need no mask for any row of the workgroup.
   int t_full0 = t_begin, t_full1 = t_end;
   if constexpr (MASK) {
     if (p.window > 0) {

@@ -240,10 +240,26 @@ __device__ __forceinline__ void map_block_kv_window(int n_tiles, int B, int Hq, 
 template <int D>
 struct DmaLayout {
   static constexpr int ROW_B = D * 2;             // bytes per K/V row
+  static constexpr int GR = 4;                    // rows per group
   static constexpr int GROUP_B = 4 * ROW_B + 16;  // 4-row group + pad
   static constexpr int LPR = ROW_B / 16;          // lanes per row in one direct load
   static constexpr int RPI = 64 / LPR;            // rows per direct load
-  static constexpr int IPG = 4 / RPI;             // direct loads per 4-row group
+  static constexpr int IPG = 4 / RPI;             // direct loads per group
+  static constexpr int NV = IPG;                  // distinct lane constants of a direct load
+  // chunk c of row sits at position c ^ swizzle(row)
+  static __device__ __forceinline__ int swizzle(int row) { return 4 * (row & 3); }
+};
+// head_dim 64: a direct load covers 8 rows of 128 bytes, so the padding of the wider rows has no place. Chunk c of row
+// sits at c ^ swizzle(row), swizzle = row bits 1, 3, 2 as bits 2, 1, 0: 16 rows of a K fragment read (one chunk each)
+// then fall on the 16 distinct 16-byte bank groups of 256 bytes, and so do the 4 rows x 4 chunks of 32 lanes of a V
+// transposing read (rows r and r + 2, on the same half, differ in chunk bit 2).
+template <>
+struct DmaLayout<64> {
+  static constexpr int ROW_B = 128, GR = 8, GROUP_B = 8 * ROW_B, LPR = 8, RPI = 8, IPG = 1;
+  static constexpr int NV = 2;  // the swizzle differs between even and odd 8-row groups
+  static __device__ __forceinline__ int swizzle(int row) {
+    return ((row >> 1) & 1) << 2 | ((row >> 3) & 1) << 1 | ((row >> 2) & 1);
+  }
 };
 
 typedef __attribute__((address_space(3))) char lds_char;

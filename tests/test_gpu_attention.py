@@ -95,6 +95,50 @@ def test_prefill_d256_gqa_large_kv_order(gpu, B, Sq, Sk, Hq, Hkv, dtype, causal,
         assert_close(out[:, :, h:h + 1].float(), ref.float(), *TOL[dtype], what)
 
 
+# Every form of the head_dim 64 / 128 forward (rows per workgroup and waves per row block, chosen by the number of
+# workgroups a launch has): heads, the few that are checked are whole. Sizes at the edges of 32-row blocks and 32 / 128-key
+# tiles, rows that see no key (Sq > Sk), tiles whose key groups are partly or wholly past the end, masks on both sides.
+FORM_HEADS = [(64, 4), (64, 60), (64, 200), (128, 8), (128, 96), (128, 288)]
+FORM_SHAPES = [
+    # Sq, Sk, causal, softcap, window, dtype
+    (200, 333, True, 0.0, 0, torch.bfloat16),
+    (300, 170, True, 0.0, 0, torch.float16),
+    (190, 190, True, 30.0, 50, torch.bfloat16),
+    (129, 257, False, 0.0, 0, torch.float16),
+    (161, 31, False, 0.0, 0, torch.bfloat16),
+    (225, 127, True, 0.0, 40, torch.float16),
+]
+
+
+@pytest.mark.parametrize("with_lse", [False, True])
+@pytest.mark.parametrize("Sq,Sk,causal,softcap,window,dtype", FORM_SHAPES)
+@pytest.mark.parametrize("D,H", FORM_HEADS)
+def test_prefill_forms(gpu, D, H, Sq, Sk, causal, softcap, window, dtype, with_lse):
+    q, k, v = _qkv(1, Sq, Sk, H, H, D, dtype, seed=Sq + Sk + D + H)
+    res = A.attention(q.to(gpu), k.to(gpu), v.to(gpu), causal=causal, softcap=softcap, window=window,
+                      return_lse=with_lse)
+    out, lse = res if with_lse else (res, None)
+    hs = [0, H // 2, H - 1]
+    ref, ref_lse = oa.attention(q[:, :, hs], k[:, :, hs], v[:, :, hs], causal=causal, softcap=softcap or None,
+                                window=window or None, return_lse=True)
+    what = f"D{D} H{H} Sq{Sq} Sk{Sk} {dtype} causal={causal} cap={softcap} win={window}"
+    assert_close(out.cpu()[:, :, hs].float(), ref.float(), *TOL[dtype], what + " out")
+    if with_lse:
+        lse_c = lse.cpu()[:, hs]
+        fin = torch.isfinite(ref_lse)
+        assert torch.equal(torch.isfinite(lse_c), fin), what + " lse -inf pattern"
+        assert_close(lse_c[fin], ref_lse[fin], 2e-2, 1e-2, what + " lse")
+
+
+def test_prefill_two_rounds_of_unequal_rows(gpu):
+    """Causal rows of one 256-row workgroup per CU at most: the 128-row form in two rounds."""
+    S, H = 1000, 40
+    q, k, v = _qkv(1, S, S, H, H, 128, torch.bfloat16, seed=5)
+    out = A.attention(q.to(gpu), k.to(gpu), v.to(gpu), causal=True).cpu()
+    ref = oa.attention(q[:, :, [0, 39]], k[:, :, [0, 39]], v[:, :, [0, 39]], causal=True)
+    assert_close(out[:, :, [0, 39]].float(), ref.float(), *TOL[torch.bfloat16], "S1000 H40")
+
+
 FAST_CASES = [
     # bf16, head_dim 128, no lse / soft-cap / reference rounding: B, Sq, Sk, Hq, Hkv, causal, window
     (1, 512, 512, 2, 2, True, 0),
