@@ -54,7 +54,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   __shared__ __attribute__((aligned(16))) S Ks[2][BN][KP];
 
   int qt, bh;
-  map_block(p.n_tiles, p.B * p.Hq, true, qt, bh);
+  map_block<true>(p.n_tiles, p.B * p.Hq, true, qt, bh);
   const int b = bh / p.Hq, h = bh - b * p.Hq;
   const int hk = h / p.group;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, r = lane & 31, g = lane >> 5;
@@ -245,6 +245,215 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   if (qi < p.Sq && g == 0) p.lse[(int64_t)bh * p.Sq + qi] = m_run == -INFINITY ? -INFINITY : m_run + fast_log2(l_tot);
 }
 
+// KeyFormer pass 1 for head_dim 128 and exp_rand rows of whole 16-byte chunks: the same reduction by 8 waves over 128
+// rows, two waves (key groups) to the same 32 rows, each taking 32 keys of every 64-key tile. K tiles and exp_rand are
+// copied global -> LDS directly. A wave's exp_rand (32 rows x 32 keys) is its own, so it needs no barrier and one buffer:
+// it is read into registers at the start of a tile and the next tile's copies follow at once. Chunk c of row r of it
+// sits at position c ^ (r / 2 % 8), so that 16 rows of one chunk are on distinct banks.
+// What bounds it: with few rows the latency of a wave's chain (products, log2, maximum, exp2: ~1 us per 32 keys, hence
+// the key groups and four waves per SIMD), with many the exp_rand stream. The tiles of a workgroup are taken from a
+// starting point of its own: rows of a power-of-two length lie on few memory channels, and workgroups that all walk the
+// columns in step keep hitting the same ones (S=2048, H=32, fp16, causal: 94.6 us without, 71.9 with; S=4096 218 / 227).
+// Against the register-staged kernel above, same calls: S=1000 35.7 -> 29.1 us, S=2048 98 -> 72, S=4096 226 / 227.
+template <typename T, bool MASK, int REFROUND>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
+attn_kf_rowlse_dma_kernel(AttnParams p) {
+  typedef typename T::scalar S;
+  typedef typename T::vec8 V8;
+  constexpr int D = 128, NW = 8, KG = 2, NWR = NW / KG, BN = 32 * KG, BM = 32 * NWR;
+  static_assert(BM == kBM, "rows per workgroup");
+  typedef DmaLayout<D> L;
+  constexpr int KT_B = (BN / 4) * L::GROUP_B;      // K tile
+  constexpr int ET_B = 32 * 32 * 4;                // one wave's exp_rand
+  constexpr int KPW = BN / 4 / NW, EPW = ET_B / 1024;  // copies per wave and tile
+  constexpr int QSLOT_B = 8 * L::GROUP_B;
+  static_assert(NWR * QSLOT_B <= 2 * KT_B, "the Q tile passes through the K ring");
+  __shared__ __attribute__((aligned(1024))) char smem[2 * KT_B + NW * ET_B];
+
+  int qt, bh;
+  map_block<true>(p.n_tiles, p.B * p.Hq, true, qt, bh);
+  const int b = bh / p.Hq, h = bh - b * p.Hq;
+  const int hk = h / p.group;
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, g = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = w % NWR, kg = w / NWR;  // row block and key group
+  const int q0 = qt * BM, qw0 = q0 + 32 * wr;
+  const int qi = qw0 + r;
+  const char* qp = reinterpret_cast<const char*>(static_cast<const S*>(p.q) + b * p.q_sb + h * p.q_sh);
+  const char* kp = reinterpret_cast<const char*>(static_cast<const S*>(p.k) + b * p.k_sb + hk * p.k_sh);
+  const int64_t q_ss_b = p.q_ss * (int64_t)sizeof(S), k_ss_b = p.k_ss * (int64_t)sizeof(S);
+  const uint32_t smem_base = (uint32_t)(size_t)((lds_char*)smem);
+  const uint32_t e_slot = smem_base + (uint32_t)(2 * KT_B + w * ET_B);
+  const int rr = lane >> 4;                                       // row of a 4-row group, in a Q / K copy
+  const uint32_t chunk_b = 16u * (uint32_t)((lane & 15) ^ L::swizzle(rr));
+
+  // Q through the K ring into registers, the two key groups copying half of a row block's rows each (rows past the end
+  // read the last row and are zeroed below).
+  const uint32_t q_slot = smem_base + (uint32_t)(wr * QSLOT_B);
+#pragma unroll
+  for (int i = 0; i < 8 / KG; ++i) {
+    const int j = KG * i + kg;
+    dma16(q_slot + j * L::GROUP_B, qp + (int64_t)min(qw0 + 4 * j + rr, p.Sq - 1) * q_ss_b + chunk_b);
+  }
+
+  const int q_last = min(q0 + BM, p.Sq) - 1;
+  int k_begin = 0, k_end = p.Sk;
+  if (p.causal) k_end = min(p.Sk, q_last + p.offset + 1);
+  if (p.window > 0) k_begin = max(0, q0 + p.offset - p.window + 1);
+  const int t_begin = k_begin / BN;
+  const int n_t = k_end > k_begin ? (k_end + BN - 1) / BN - t_begin : 0;
+  const int rot = n_t > 0 ? (int)((blockIdx.x >> 3) * 7 % n_t) : 0;
+  auto tile_of = [&](int i) { return t_begin + (i + rot < n_t ? i + rot : i + rot - n_t); };
+  int k_hi = p.Sk - 1, k_lo = 0;
+  if (p.causal) k_hi = min(k_hi, qi + p.offset);
+  if (p.window > 0) k_lo = max(k_lo, qi + p.offset - p.window + 1);
+
+  // exp_rand copy i of a tile: rows 8i + lane / 8 of the wave, position lane % 8 of the row. Where every row and key
+  // exists: a scalar address plus one of two lane offsets (the swizzle of rows 8i.. differs between even and odd i).
+  // At the edges: the last row, the last whole chunk of exp_rand, the last key of K (masked, finite: exactly 0).
+  const char* eb = reinterpret_cast<const char*>(p.er + b * p.er_sb + h * p.er_sh);
+  const int64_t er_ss_b = p.er_ss * 4;
+  const bool rows_ok = qw0 + 32 <= p.Sq && p.er_lane32;
+  uint32_t e_voff[2], k_voff = (uint32_t)(rr * k_ss_b) + chunk_b;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    e_voff[i] = (uint32_t)((lane >> 3) * er_ss_b) + 16u * (uint32_t)((lane & 7) ^ ((4 * i + (lane >> 4)) & 7));
+  auto issue_e = [&](int t) __attribute__((always_inline)) {
+    const int kb = t * BN + 32 * kg;
+    if (rows_ok && kb + 32 <= p.Sk) {
+      const char* base = eb + (int64_t)qw0 * er_ss_b + (int64_t)kb * 4;
+#pragma unroll
+      for (int i = 0; i < EPW; ++i) dma16(e_slot + 1024 * i, base + 8 * i * er_ss_b, e_voff[i & 1]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < EPW; ++i) {
+        const int row = 8 * i + (lane >> 3), col = kb + 4 * ((lane & 7) ^ ((row >> 1) & 7));
+        dma16(e_slot + 1024 * i, eb + ((int64_t)min(qw0 + row, p.Sq - 1) * p.er_ss + min(col, p.Sk - 4)) * 4);
+      }
+    }
+  };
+  auto issue_k = [&](int slot, int t) __attribute__((always_inline)) {
+    const uint32_t dst = smem_base + (uint32_t)((slot & 1) * KT_B + KPW * w * L::GROUP_B);
+    if ((t + 1) * BN <= p.Sk) {
+      const char* base = kp + (int64_t)(t * BN + 4 * KPW * w) * k_ss_b;
+#pragma unroll
+      for (int j = 0; j < KPW; ++j) dma16(dst + j * L::GROUP_B, base + 4 * j * k_ss_b, k_voff);
+    } else {
+#pragma unroll
+      for (int j = 0; j < KPW; ++j)
+        dma16(dst + j * L::GROUP_B, kp + (int64_t)min(t * BN + 4 * (KPW * w + j) + rr, p.Sk - 1) * k_ss_b + chunk_b);
+    }
+  };
+
+  const int s4 = r & 3;
+  uint32_t xq[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) xq[i] = (uint32_t)((r >> 2) * L::GROUP_B + s4 * L::ROW_B + 16 * g + 64 * (i ^ s4));
+  if (n_t > 0) issue_e(tile_of(0));
+  V8 qf[D / 16];
+  if (n_t > 0) wait_vmem<EPW>();
+  else wait_vmem<0>();
+  __syncthreads();
+#pragma unroll
+  for (int kk = 0; kk < D / 16; ++kk) qf[kk] = lds_read<V8>(q_slot + xq[kk >> 1] + 32 * (kk & 1));
+#pragma unroll
+  for (int kk = 0; kk < D / 16; ++kk) {
+    asm volatile("" : "+v"(qf[kk]));
+    if (qi >= p.Sq) qf[kk] = V8{};
+  }
+  __syncthreads();  // every wave has its Q: the ring is free
+  if (n_t > 0) issue_k(0, tile_of(0));
+
+  // fp16 reference rounding keeps each pair of scores packed (two instructions per score instead of four)
+  constexpr bool PK = REFROUND && std::is_same<T, F16>::value;
+  const float cy = (PK ? kLog2e : score_coeff<false, REFROUND>(p)) * p.kf_inv_tau;  // score -> exp2 domain / tau
+  float m_run = -INFINITY, l_run = 0.f;
+  auto tile = [&](int t, f32x16& sacc, const f32x4 (&ev)[4], auto masked) __attribute__((always_inline)) {
+    // element j holds key t*BN + 32*kg + 8*(j/4) + 4g + j%4
+    const int kb4 = t * BN + 32 * kg + 4 * g;
+    const int rel_hi = k_hi - kb4, rel_lo = k_lo - kb4;
+    float mloc = -INFINITY;
+    f16x2 hpair;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      // y = (x2 - log2 e) / tau as one fma of the score against per-launch constants: the score x in the natural log
+      // domain times log2(e) / tau (PK: the reference-rounded fp16 pair, read by v_fma_mix), or x * c / tau
+      float x;
+      if constexpr (PK) {
+        if ((j & 1) == 0) hpair = ref_scores_f16(sacc[j], sacc[j + 1], p);
+        x = (float)hpair[j & 1];
+      } else {
+        x = score_value<T, false, REFROUND>(sacc[j], p);
+      }
+      float y = fmaf(x, cy, -fast_log2(ev[j >> 2][j & 3]) * p.kf_inv_tau);
+      const int o = 8 * (j >> 2) + (j & 3);
+      if constexpr (decltype(masked)::value) y = (o <= rel_hi && o >= rel_lo) ? y : -INFINITY;
+      sacc[j] = y;
+      mloc = fmaxf(mloc, y);
+    }
+    mloc = half_swap_max(mloc);
+    const float m_new = fmaxf(m_run, mloc);
+    if (m_new > m_run + kRescaleThreshold || (m_run == -INFINITY && m_new > -INFINITY)) {
+      l_run *= fast_exp2(m_run - m_new);  // 0 while m_run is -inf
+      m_run = m_new;
+    }
+    const float mu = m_run == -INFINITY ? 0.f : m_run;
+    float part[2] = {0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 16; ++j) part[j & 1] += fast_exp2(sacc[j] - mu);
+    l_run += part[0] + part[1];
+  };
+
+  // Keys [wk_begin, wk_end) are seen by some row of this wave, [f0, f1) by every one.
+  int wk_begin = 0, wk_end = qw0 < p.Sq ? p.Sk : 0, f0 = 0, f1 = p.Sk;
+  if constexpr (MASK) {
+    const int wq_last = min(qw0 + 32, p.Sq) - 1;
+    if (p.window > 0) {
+      wk_begin = max(0, qw0 + p.offset - p.window + 1);
+      f0 = max(0, wq_last + p.offset - p.window + 1);
+    }
+    if (p.causal) {
+      wk_end = min(wk_end, wq_last + p.offset + 1);
+      f1 = min(f1, qw0 + p.offset + 1);
+    }
+  }
+  for (int i = 0; i < n_t; ++i) {
+    wait_vmem<0>();
+    __syncthreads();  // tile i of K is in the LDS; every wave has left tile i - 1
+    if (i + 1 < n_t) issue_k(i + 1, tile_of(i + 1));
+    const int t = tile_of(i), kb = t * BN + 32 * kg;
+    const bool live = kb < wk_end && kb + 32 > wk_begin;
+    f32x16 sacc = f32x16{};
+    if (live) {
+      const uint32_t st = smem_base + (uint32_t)((i & 1) * KT_B + kg * (KT_B / KG));
+#pragma unroll
+      for (int kk = 0; kk < D / 16; ++kk) sacc = mfma32(lds_read<V8>(st + xq[kk >> 1] + 32 * (kk & 1)), qf[kk], sacc);
+    }
+    // exp_rand after the products (fewer registers at once: 128 are what four waves per SIMD have)
+    f32x4 ev[4];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int jq = 0; jq < 4; ++jq) ev[jq] = lds_read<f32x4>(e_slot + r * 128 + 16 * ((2 * jq + g) ^ ((r >> 1) & 7)));
+#pragma unroll
+    for (int jq = 0; jq < 4; ++jq) asm volatile("" : "+v"(ev[jq]));  // read: the buffer may be overwritten
+    if (i + 1 < n_t) issue_e(tile_of(i + 1));
+    if (!live) continue;
+    if (kb >= f0 && kb + 32 <= f1) tile(t, sacc, ev, std::false_type{});
+    else tile(t, sacc, ev, std::true_type{});
+  }
+  float l_tot = half_swap_sum(l_run);
+  __syncthreads();  // the ring is done with
+  f32x2* ml = reinterpret_cast<f32x2*>(smem);  // key group 1's (maximum, sum) per row
+  if (kg == 1 && g == 0) ml[32 * wr + r] = f32x2{m_run, l_tot};
+  __syncthreads();
+  if (kg == 0 && g == 0 && qi < p.Sq) {
+    const f32x2 o = ml[32 * wr + r];
+    const float m = fmaxf(m_run, o[0]), mu = m == -INFINITY ? 0.f : m;
+    l_tot = l_tot * fast_exp2(m_run - mu) + o[1] * fast_exp2(o[0] - mu);
+    p.lse[(int64_t)bh * p.Sq + qi] = m == -INFINITY ? -INFINITY : m + fast_log2(l_tot);
+  }
+}
+
 // ------------------------------------------------------------------------------------------------
 // Column-sum kernel: colsum[b,h,j] = sum_i exp(score_ij - lse_i). A workgroup owns 128 keys (32 per wave,
 // held in VGPRs as the B operand); query tiles of 64 rows stream through double-buffered LDS together
@@ -409,19 +618,20 @@ __device__ __forceinline__ void dma4(uint32_t lds, const void* vaddr) {
                : "memory", "m0");
 }
 
-// KPW: 32-key blocks per wave. With two, each Q fragment read from the LDS feeds two MFMAs (one per key block).
-template <typename T, int NW, int KPW, int BQ, int NSTAGE, bool MASK, bool SOFTCAP, int REFROUND, bool LSE2, int EPI>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
+// NG: row groups of NW / NG waves. Each group covers every key of the workgroup (32 * NW / NG keys) and takes its own
+// BQ / NG rows of each query tile; the groups' results are combined through the LDS at the end. OCC: waves per SIMD the
+// register budget is sized for (4: two workgroups per CU, whose LDS fits).
+template <typename T, int NW, int NG, int BQ, int OCC, bool MASK, bool SOFTCAP, int REFROUND, bool LSE2, int EPI>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 attn_colsum_d128_kernel(AttnParams p) {
   constexpr int D = 128;
   constexpr int ROW_B = DmaLayout<D>::ROW_B, GROUP_B = DmaLayout<D>::GROUP_B;
   typedef typename T::scalar S;
   typedef typename T::vec8 V8;
-  // With KPW key blocks per wave the waves form KPW row groups of NW / KPW waves: each group covers every key of
-  // the workgroup and takes its own BQ / KPW rows of each query tile; the groups' sums are added at the end.
-  constexpr int NG = KPW, NWG = NW / NG;     // row groups, waves per group
+  constexpr int NWG = NW / NG;               // waves per row group
   constexpr int BQW = BQ / NG;               // query rows of a tile per row group
-  constexpr int BK = 32 * KPW * NWG;         // keys per workgroup
+  constexpr int BK = 32 * NWG;               // keys per workgroup
+  constexpr int NSTAGE = 2;                  // query tiles in the LDS ring
   constexpr int QT_B = (BQ / 4) * GROUP_B;   // bytes of one Q tile
   constexpr int STAGE_B = QT_B + 4 * BQ;     // Q tile, then its BQ lse values
   constexpr int GPW = (BQ / 4) / NW;         // 4-row groups of a Q tile copied by each wave
@@ -429,13 +639,13 @@ attn_colsum_d128_kernel(AttnParams p) {
   constexpr int NMB = BQW / 32;              // 32-row query blocks of a wave's part of a tile
   static_assert(GPW >= 1 && GPW * NW == BQ / 4, "Q tile groups must split over the waves");
   static_assert(BQ % 64 == 0 && QT_B % 16 == 0 && BQW % 32 == 0 && NWG * NG == NW, "tile shape");
-  static_assert(KPW == 1 || ((EPI == kColSum || EPI == kColSumSq) && KPW == 2), "two key blocks: sum epilogues");
-  static_assert(NG == 1 || NSTAGE * STAGE_B >= 4 * 2 * BK, "the groups' sums are combined in the LDS");
-  constexpr int NSB = KPW * NMB;  // score blocks of a tile: block kp * NMB + mb (key block kp, query block mb)
+  static_assert(NG == 1 || NSTAGE * STAGE_B >= (NG - 1) * 2 * BK * 4, "the groups' sums are combined in the LDS");
+  constexpr int KSLOT_B = 8 * GROUP_B;  // 32 keys on their way to the registers
+  static_assert(NWG * KSLOT_B <= STAGE_B, "the workgroup's keys pass through the stage that no first copy fills");
   __shared__ __attribute__((aligned(1024))) char smem[NSTAGE * STAGE_B];
 
   int kt, bh;
-  map_block(p.n_tiles, p.B * p.Hq, false, kt, bh);
+  map_block<OCC == 4>(p.n_tiles, p.B * p.Hq, false, kt, bh);
   const int b = bh / p.Hq, h = bh - b * p.Hq;
   const int hk = h / p.group;
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, g = lane >> 5;
@@ -443,27 +653,13 @@ attn_colsum_d128_kernel(AttnParams p) {
   const int wi = w % NWG, gw = w / NWG;  // wave within its row group, row group
   const int rg0 = BQW * gw;              // first row of the group's part of a query tile
   const int k0 = kt * BK;
-  const int kw0 = k0 + 32 * KPW * wi;  // first key of this wave
-  const int kj = kw0 + r;             // this lane's key (of key block 0; block kp: kj + 32 kp)
+  const int kw0 = k0 + 32 * wi;  // first key of this wave
+  const int kj = kw0 + r;             // this lane's key
 
   const S* kp = static_cast<const S*>(p.k) + b * p.k_sb + hk * p.k_sh;
   const char* qp = reinterpret_cast<const char*>(static_cast<const S*>(p.q) + b * p.q_sb + h * p.q_sh);
   const int64_t q_ss_b = p.q_ss * (int64_t)sizeof(S);
   const float* lsep = p.lse + (int64_t)bh * p.Sq;
-
-  V8 kf[KPW][D / 16];
-#pragma unroll
-  for (int kb = 0; kb < KPW; ++kb)
-#pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk)  // back-to-back loads (keys past the end read the last key, zeroed below)
-      kf[kb][kk] = ld16<V8>(kp + (int64_t)min(kj + 32 * kb, p.Sk - 1) * p.k_ss + 16 * kk + 8 * g);
-#pragma unroll
-  for (int kb = 0; kb < KPW; ++kb)
-#pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
-      asm volatile("" : "+v"(kf[kb][kk]));  // see the forward kernel
-      if (kj + 32 * kb >= p.Sk) kf[kb][kk] = V8{};
-    }
 
   // Query tiles that see any key of the workgroup, and of this wave.
   const int k_last = min(k0 + BK, p.Sk) - 1;
@@ -474,7 +670,7 @@ attn_colsum_d128_kernel(AttnParams p) {
   const int t_end = q_end > q_begin ? (q_end + BQ - 1) / BQ : t_begin;
   int wt_begin = t_begin, wt_end = t_begin;  // empty for a wave whose keys all lie past Sk
   if (kw0 < p.Sk) {
-    const int wk_last = min(kw0 + 32 * KPW, p.Sk) - 1;
+    const int wk_last = min(kw0 + 32, p.Sk) - 1;
     int wq_begin = 0, wq_end = p.Sq;
     if (p.causal) wq_begin = max(0, kw0 - p.offset);
     if (p.window > 0) wq_end = min(p.Sq, wk_last - p.offset + p.window);
@@ -486,11 +682,11 @@ attn_colsum_d128_kernel(AttnParams p) {
       if (wt_end < wt_begin) wt_end = wt_begin;
     }
   }
-  // Tiles [t_full0, t_full1) need no mask for this wave: every row < Sq of its part sees all of its 32 * KPW keys.
+  // Tiles [t_full0, t_full1) need no mask for this wave: every row < Sq of its part sees all of its 32 keys.
   int t_full0 = t_begin, t_full1 = t_end;
   if constexpr (MASK) {
     if (p.causal) {
-      const int a = kw0 + 32 * KPW - 1 - p.offset - rg0;  // first row that sees the wave's last key, less rg0
+      const int a = kw0 + 32 - 1 - p.offset - rg0;  // first row that sees the wave's last key, less rg0
       t_full0 = a <= 0 ? t_begin : min(t_end, max(t_begin, (a + BQ - 1) / BQ));
     }
     if (p.window > 0) {
@@ -532,6 +728,17 @@ attn_colsum_d128_kernel(AttnParams p) {
     }
   };
 
+  // The keys: copied like the Q tiles (a fragment load straight from global memory has 64 lanes on 32 rows, ~64 cycles
+  // of address processing each), the row groups taking turns at the 4-row groups of a slot. Keys past the end read the
+  // last key and are zeroed.
+  const uint32_t kslot = smem_base + (uint32_t)(((t_begin + NSTAGE - 1) % NSTAGE) * STAGE_B + wi * KSLOT_B);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    if (NG > 1 && j % NG != gw) continue;
+    const int64_t key = min(kw0 + 4 * j + rr, p.Sk - 1);
+    dma16(kslot + j * GROUP_B, reinterpret_cast<const char*>(kp + key * p.k_ss) + src_chunk * 16);
+  }
+
   // Q fragment (row 32mb + r, chunk 2kk + g) addressing, as the forward's K fragments.
   const int s4 = r & 3;
   const uint32_t q_lane = (uint32_t)((rg0 / 4 + (r >> 2)) * GROUP_B + s4 * ROW_B + 16 * g);
@@ -542,7 +749,7 @@ attn_colsum_d128_kernel(AttnParams p) {
   constexpr bool PK = REFROUND && !SOFTCAP && std::is_same<T, F16>::value;
   const float c = PK ? kLog2e : score_coeff<SOFTCAP, REFROUND>(p);
   const float cy = EPI == kColKF ? c * p.kf_inv_tau : 0.f;  // KeyFormer: score -> exp2 domain / tau
-  ColAcc<EPI> acc[KPW];
+  ColAcc<EPI> acc;
   const int kjc = min(kj, p.Sk - 1);
   const float* erp = EPI == kColKF ? p.er + b * p.er_sb + h * p.er_sh : nullptr;  // KeyFormer exp_rand of (b, h)
   // KeyFormer exp_rand of (row, kjc) for tiles whose rows all exist: a wave-uniform tile address (scalar registers)
@@ -551,52 +758,44 @@ attn_colsum_d128_kernel(AttnParams p) {
   // Corm's thresholds of (row, kjc), addressed the same way.
   const uint32_t thr_lane_b = EPI == kColAnyGe ? (uint32_t)((4 * g * p.thr_rs + kjc) * 4) : 0u;
 
+  V8 kf[D / 16];  // this wave's keys (B operand), read below
   // S = Q . K^T of query tile t (its LDS stage) into s.
-  auto qk_t = [&](const int t, f32x16 (&s)[NSB]) __attribute__((always_inline)) {
+  auto qk_t = [&](const int t, f32x16 (&s)[NMB]) __attribute__((always_inline)) {
     const uint32_t st = smem_base + (uint32_t)((t % NSTAGE) * STAGE_B);
-    uint32_t qb[4];  // opaque per-stage bases (reads at base + immediate offset)
+    uint32_t qb[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      qb[i] = st + xq[i];
-      if constexpr (NSTAGE == 3) asm volatile("" : "+v"(qb[i]));
-    }
+    for (int i = 0; i < 4; ++i) qb[i] = st + xq[i];
 #pragma unroll
-    for (int i = 0; i < NSB; ++i) s[i] = f32x16{};
+    for (int i = 0; i < NMB; ++i) s[i] = f32x16{};
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
+    for (int kk = 0; kk < D / 16; ++kk)
 #pragma unroll
       for (int mb = 0; mb < NMB; ++mb) {
         const V8 a = lds_read<V8>(qb[kk >> 1] + mb * 8 * GROUP_B + 32 * (kk & 1));
-#pragma unroll
-        for (int kb = 0; kb < KPW; ++kb) s[kb * NMB + mb] = mfma32(a, kf[kb][kk], s[kb * NMB + mb]);
+        s[mb] = mfma32(a, kf[kk], s[mb]);
       }
-    }
   };
-  auto epi_t = [&](const int t, const f32x16 (&sacc)[NSB], const float (&ev)[NMB][16], const float (&tv)[NMB][16],
+  auto epi_t = [&](const int t, const f32x16 (&sacc)[NMB], const float (&ev)[NMB][16], const float (&tv)[NMB][16],
                    auto masked) __attribute__((always_inline)) {
-    uint32_t lb = smem_base + (uint32_t)((t % NSTAGE) * STAGE_B) + QT_B + 4 * rg0 + 16 * g;  // this lane's lse
-    if constexpr (NSTAGE == 3) asm volatile("" : "+v"(lb));
+    const uint32_t lb = smem_base + (uint32_t)((t % NSTAGE) * STAGE_B) + QT_B + 4 * rg0 + 16 * g;  // this lane's lse
     // Visibility of (row o of the tile, this lane's key): causal rel >= 0, window rel < window, row < Sq.
     const int rows_left = p.Sq - t * BQ - rg0 - 4 * g;
+    const int rel0 = t * BQ + rg0 + 4 * g + p.offset - kj;
 #pragma unroll
     for (int mb = 0; mb < NMB; ++mb) {
       f32x4 lv[4];
 #pragma unroll
       for (int jq = 0; jq < 4; ++jq) lv[jq] = lds_read<f32x4>(lb + 4 * (32 * mb + 8 * jq));
-#pragma unroll
-      for (int kb = 0; kb < KPW; ++kb) {
-      const f32x16& sb = sacc[kb * NMB + mb];
-      const int rel0 = t * BQ + rg0 + 4 * g + p.offset - (kj + 32 * kb);
       f16x2 hs[8];
       if constexpr (PK) {
 #pragma unroll
-        for (int jp = 0; jp < 8; ++jp) hs[jp] = ref_scores_f16(sb[2 * jp], sb[2 * jp + 1], p);
+        for (int jp = 0; jp < 8; ++jp) hs[jp] = ref_scores_f16(sacc[mb][2 * jp], sacc[mb][2 * jp + 1], p);
       }
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         float x;
         if constexpr (PK) x = (float)hs[j >> 1][j & 1];
-        else x = score_value<T, SOFTCAP, REFROUND>(sb[j], p);
+        else x = score_value<T, SOFTCAP, REFROUND>(sacc[mb][j], p);
         const float l2 = LSE2 ? lv[j >> 2][j & 3] : lv[j >> 2][j & 3] * kLog2e;
         const int o = 32 * mb + 8 * (j >> 2) + (j & 3);
         float pe;
@@ -616,9 +815,8 @@ attn_colsum_d128_kernel(AttnParams p) {
           vis = ok;
         }
         // Corm compares visible pairs here; the masked ones (p = 0) are ORed in by corm_masked_or_kernel
-        if constexpr (EPI == kColAnyGe) acc[0].any |= vis && pe >= tv[mb][j];
-        else acc[kb].add(pe, valid, min(t * BQ + rg0 + 4 * g + o, p.Sq - 1), min(kjc + 32 * kb, p.Sk - 1), p);
-      }
+        if constexpr (EPI == kColAnyGe) acc.any |= vis && pe >= tv[mb][j];
+        else acc.add(pe, valid, min(t * BQ + rg0 + 4 * g + o, p.Sq - 1), kjc, p);
       }
     }
   };
@@ -627,7 +825,7 @@ attn_colsum_d128_kernel(AttnParams p) {
     float ev[NMB][16];
     if constexpr (EPI == kColKF) {
       if constexpr (!decltype(masked)::value) {  // every row of the tile exists (and er_lane32 holds)
-        const char* rb = reinterpret_cast<const char*>(erp + (int64_t)(t * BQ) * p.er_ss);
+        const char* rb = reinterpret_cast<const char*>(erp + (int64_t)(t * BQ + rg0) * p.er_ss);
         uint32_t ss_b = (uint32_t)(p.er_ss * 4);
         asm volatile("" : "+s"(ss_b));  // per tile: keeps the 64 offsets from being hoisted into registers
 #pragma unroll
@@ -642,7 +840,7 @@ attn_colsum_d128_kernel(AttnParams p) {
         for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
           for (int j = 0; j < 16; ++j)
-            ev[mb][j] = erp[(int64_t)min(t * BQ + 4 * g + 32 * mb + 8 * (j >> 2) + (j & 3), p.Sq - 1) * p.er_ss + kjc];
+            ev[mb][j] = erp[(int64_t)min(t * BQ + rg0 + 4 * g + 32 * mb + 8 * (j >> 2) + (j & 3), p.Sq - 1) * p.er_ss + kjc];
       }
     }
     // Corm: the tile's thresholds for this lane's key, requested before the QK^T MFMAs so that the loads overlap
@@ -650,7 +848,7 @@ attn_colsum_d128_kernel(AttnParams p) {
     float tv[NMB][16];
     if constexpr (EPI == kColAnyGe) {
       if constexpr (!decltype(masked)::value) {  // every row of the tile exists (and thr_lane32 holds)
-        const char* rb = reinterpret_cast<const char*>(p.thr + (int64_t)(t * BQ) * p.thr_rs);
+        const char* rb = reinterpret_cast<const char*>(p.thr + (int64_t)(t * BQ + rg0) * p.thr_rs);
         uint32_t ss_b = (uint32_t)(p.thr_rs * 4);
         asm volatile("" : "+s"(ss_b));  // per tile: keeps the 64 offsets from being hoisted into registers
 #pragma unroll
@@ -665,10 +863,10 @@ attn_colsum_d128_kernel(AttnParams p) {
         for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
           for (int j = 0; j < 16; ++j)
-            tv[mb][j] = p.thr[(int64_t)min(t * BQ + 4 * g + 32 * mb + 8 * (j >> 2) + (j & 3), p.Sq - 1) * p.thr_rs + kjc];
+            tv[mb][j] = p.thr[(int64_t)min(t * BQ + rg0 + 4 * g + 32 * mb + 8 * (j >> 2) + (j & 3), p.Sq - 1) * p.thr_rs + kjc];
       }
     }
-    f32x16 sacc[NSB];
+    f32x16 sacc[NMB];
     qk_t(t, sacc);
     epi_t(t, sacc, ev, tv, masked);
   };
@@ -676,107 +874,36 @@ attn_colsum_d128_kernel(AttnParams p) {
 #pragma unroll
   for (int i = 0; i < NSTAGE - 1; ++i)
     if (t_begin + i < t_end) issue(t_begin + i);
+  // The key fragments, once their copies have landed (those of the first Q tile may stay in flight; the last wave
+  // issued NLSE more of them).
+  if (t_begin >= t_end) wait_vmem<0>();
+  else if (w == NW - 1) wait_vmem<GPW + NLSE>();
+  else wait_vmem<GPW>();
+  if constexpr (NG > 1) __syncthreads();
+#pragma unroll
+  for (int kk = 0; kk < D / 16; ++kk)
+    kf[kk] = lds_read<V8>(kslot + (uint32_t)((r >> 2) * GROUP_B + s4 * ROW_B + 16 * g) + 64 * ((kk >> 1) ^ s4) +
+                          32 * (kk & 1));
+#pragma unroll
+  for (int kk = 0; kk < D / 16; ++kk) {
+    asm volatile("" : "+v"(kf[kk]));
+    if (kj >= p.Sk) kf[kk] = V8{};
+  }
   // Corm: whether this wave's keys are all decided (no tile of its range left, or every key flagged).
   bool wave_done = wt_begin >= wt_end;
-  // One pipelined step: the mask-free epilogue of tile t (scores in sc) and S of tile t+1 (into sn), in a fixed
-  // order of 32 fenced steps, one per MFMA. Step i runs the QK^T MFMA of Q fragment f = i / KPW (k-step f / NMB,
-  // query block f % NMB) with key block i % KPW, reads a later fragment when it starts a fragment, and takes the
-  // exponentials and sums of score pair q = i / KPW (pair q % 8 of query block q / 8) of that key block; the lse
-  // values of the next four rows are read when a group of two pairs starts. (Left to the compiler, the fragment
-  // reads move to the front and the form spills.)
-  auto pipe_step = [&](const int t, const f32x16 (&sc)[NSB], f32x16 (&sn)[NSB]) __attribute__((always_inline)) {
-    static_assert(NSB == 4, "32 steps: 8 k-steps x 4 score blocks, 4 score blocks x 8 score pairs");
-    constexpr int NF = 32 / KPW;       // Q fragments of a tile
-    constexpr int NLG = 16 / KPW;      // groups of two score pairs (four rows' lse values) per key block
-    const uint32_t stc = smem_base + (uint32_t)((t % NSTAGE) * STAGE_B);
-    const uint32_t stn = smem_base + (uint32_t)(((t + 1) % NSTAGE) * STAGE_B);
-    // per-stage base registers, opaque to the compiler, so that every read is base + immediate offset
-    uint32_t qb[4], lb = stc + QT_B + 4 * rg0 + 16 * g;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      qb[i] = stn + xq[i];
-      asm volatile("" : "+v"(qb[i]));
-    }
-    asm volatile("" : "+v"(lb));
-    auto qread = [&](const int f) __attribute__((always_inline)) {
-      const int kk = f / NMB, mb = f % NMB;
-      return lds_read<V8>(qb[kk >> 1] + mb * 8 * GROUP_B + 32 * (kk & 1));
-    };
-    auto lread = [&](const int lg) __attribute__((always_inline)) {  // lse of the rows of pairs 2lg, 2lg+1
-      return lds_read<f32x4>(lb + 4 * (32 * (lg >> 2) + 8 * (lg & 3)));
-    };
-#pragma unroll
-    for (int i = 0; i < NSB; ++i) sn[i] = f32x16{};
-    // Q fragment ring of NA slots: fragment f + NA - 1 is read when fragment f starts, two steps before its first
-    // MFMA either way (one key block: three slots, two fragments ahead; two key blocks: two slots, one fragment
-    // ahead, each fragment feeding two steps)
-    constexpr int NA = KPW == 2 ? 2 : 3;
-    V8 a[NA];
-    f32x4 lvb[2];
-#pragma unroll
-    for (int j = 0; j < NA - 1; ++j) a[j] = qread(j);
-    lvb[0] = lread(0);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
-      const int f = i / KPW, kb = i % KPW;
-      if (kb == 0 && f + NA - 1 < NF) a[(f + NA - 1) % NA] = qread(f + NA - 1);
-      const int q = i / KPW, lg = q >> 1;
-      if (i % (2 * KPW) == 0 && lg + 1 < NLG) lvb[(lg + 1) & 1] = lread(lg + 1);
-      sn[kb * NMB + f % NMB] = mfma32(a[f % NA], kf[kb][f / NMB], sn[kb * NMB + f % NMB]);
-      const int mb = q >> 3, jp = q & 7;
-      const f32x16& sp = sc[kb * NMB + mb];
-      const f32x4& lv = lvb[lg & 1];
-      float x[2];
-      if constexpr (PK) {
-        const f16x2 hs = ref_scores_f16(sp[2 * jp], sp[2 * jp + 1], p);
-        x[0] = (float)hs[0];
-        x[1] = (float)hs[1];
-      } else {
-        x[0] = score_value<T, SOFTCAP, REFROUND>(sp[2 * jp], p);
-        x[1] = score_value<T, SOFTCAP, REFROUND>(sp[2 * jp + 1], p);
-      }
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const float l2 = LSE2 ? lv[2 * (jp & 1) + e] : lv[2 * (jp & 1) + e] * kLog2e;
-        acc[kb].add(fast_exp2(fmaf(x[e], c, -l2)), true, 0, kjc, p);
-      }
-#pragma unroll
-      for (int k2 = 0; k2 < KPW; ++k2) acc[k2].pin();
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-
-  // PIPE: the mask-free tiles of a wave run software-pipelined, the QK^T MFMAs of tile t+1 in the same basic block
-  // as the exponentials and sums of tile t (which are VALU work the MFMA pipe would otherwise wait out). Tile t+1
-  // must then be in the LDS at the barrier of tile t, so every barrier waits for all copies issued before it, and
-  // a third stage keeps tile t (its lse values) while tile t+2 lands.
-  constexpr bool PIPE = NSTAGE == 3;
-  static_assert(!PIPE || EPI == kColSum || EPI == kColSumSq, "three stages only for the pipelined epilogues");
-  // Waits for the copies of tile t (PIPE: and of tile t+1), then the barrier after which tile t+NSTAGE-1 is
-  // requested into the stage of tile t-1 (every wave has finished with it).
+  // Waits for the copies of tile t, then the barrier after which tile t+1 is requested into the stage of tile t-1
+  // (every wave has finished with it).
   auto sync = [&](const int t) -> bool {
-    // Tiles t+1 .. t+after may stay in flight; the last wave issues NLSE more copies per tile.
-    const int after = PIPE ? 0 : min(NSTAGE - 2, t_end - 1 - t);
-    if (w == NW - 1) {
-      if (NSTAGE >= 4 && after >= 2) wait_vmem<2 * (GPW + NLSE)>();
-      else if (NSTAGE >= 3 && after >= 1) wait_vmem<GPW + NLSE>();
-      else wait_vmem<0>();
-    } else {
-      if (NSTAGE >= 4 && after >= 2) wait_vmem<2 * GPW>();
-      else if (NSTAGE >= 3 && after >= 1) wait_vmem<GPW>();
-      else wait_vmem<0>();
-    }
+    wait_vmem<0>();
     if constexpr (EPI == kColAnyGe) {
       // Corm ORs over the query rows: once every key of every wave is flagged, no later tile can change the
       // result, and the workgroup stops. The vote doubles as the tile's barrier; the copies of this tile have
-      // landed and none is in flight yet (NSTAGE 2), so nothing still writes into the LDS when it stops.
-      static_assert(EPI != kColAnyGe || NSTAGE == 2, "the early stop assumes no copy in flight at the barrier");
+      // landed and none is in flight yet, so nothing still writes into the LDS when it stops.
       if (__syncthreads_and(wave_done)) return false;
     } else {
       __syncthreads();
     }
-    if (t + NSTAGE - 1 < t_end) issue(t + NSTAGE - 1);
+    if (t + 1 < t_end) issue(t + 1);
     return true;
   };
   auto step = [&](const int t, auto masked) -> bool {
@@ -785,7 +912,7 @@ attn_colsum_d128_kernel(AttnParams p) {
       tile(t, masked);
       if constexpr (EPI == kColAnyGe) {
         // this lane's key is decided when either half of its rows flagged it (keys past the end count as decided)
-        const bool decided = (acc[0].any | __shfl_xor(acc[0].any, 32, 64)) != 0 || kj >= p.Sk;
+        const bool decided = (acc.any | __shfl_xor(acc.any, 32, 64)) != 0 || kj >= p.Sk;
         wave_done = t + 1 >= wt_end || __all(decided);
       }
     }
@@ -793,101 +920,84 @@ attn_colsum_d128_kernel(AttnParams p) {
   };
   bool go = true;
   for (int t = t_begin; go && t < t_full0; ++t) go = step(t, std::true_type{});
-  // The mask-free range lies inside the wave's range whenever the wave has keys (kw0 < Sk).
-  if (PIPE && t_full1 - t_full0 >= 2 && t_full0 >= wt_begin && t_full1 <= wt_end) {
-    // scores of two tiles in flight, in two buffers that swap roles every step (loop unrolled by two)
-    f32x16 sa[NSB], sb[NSB];
-    float none[NMB][16];  // KeyFormer / Corm inputs, never read by these epilogues
-    int t = t_full0;
-    sync(t);
-    qk_t(t, sa);
-    pipe_step(t, sa, sb);
-    for (++t;;) {
-      sync(t);
-      if (t + 1 >= t_full1) {
-        epi_t(t, sb, none, none, std::false_type{});
-        break;
-      }
-      pipe_step(t, sb, sa);
-      sync(++t);
-      if (t + 1 >= t_full1) {
-        epi_t(t, sa, none, none, std::false_type{});
-        break;
-      }
-      pipe_step(t, sa, sb);
-      ++t;
-    }
-  } else {
-    for (int t = t_full0; go && t < t_full1; ++t) go = step(t, std::false_type{});
-  }
+  for (int t = t_full0; go && t < t_full1; ++t) go = step(t, std::false_type{});
   for (int t = t_full1; go && t < t_end; ++t) go = step(t, std::true_type{});
 
   if constexpr (NG == 1) {
-    acc[0].store(p, bh, kj, g);
+    acc.store(p, bh, kj, g);
   } else {
-    // Row group 1 leaves its sums (lane halves added) in the LDS; group 0 adds them to its own and stores.
+    // Row groups 1 .. leave their results (lane halves combined) in the LDS; group 0 combines them with its own, in
+    // group order, and stores.
     wait_vmem<0>();
     __syncthreads();  // every wave is done with the Q stages
-    float* red = reinterpret_cast<float*>(smem);
-#pragma unroll
-    for (int kb = 0; kb < KPW; ++kb) {
-      acc[kb].s += __shfl_xor(acc[kb].s, 32, 64);
-      if constexpr (EPI == kColSumSq) acc[kb].s2 += __shfl_xor(acc[kb].s2, 32, 64);
-      const int key = 32 * (KPW * wi + kb) + r;  // key within the workgroup
-      if (gw == 1 && g == 0) {
-        red[key] = acc[kb].s;
-        if constexpr (EPI == kColSumSq) red[BK + key] = acc[kb].s2;
-      }
+    float* red = reinterpret_cast<float*>(smem);  // [group - 1][2][BK]
+    const int key = 32 * wi + r;                  // key within the workgroup
+    if constexpr (EPI == kColAnyGe) {
+      acc.any |= __shfl_xor(acc.any, 32, 64);
+    } else {
+      acc.s += __shfl_xor(acc.s, 32, 64);
+      if constexpr (EPI == kColSumSq) acc.s2 += __shfl_xor(acc.s2, 32, 64);
+    }
+    float t1 = EPI == kColAnyGe ? (acc.any ? 1.0f : 0.0f) : acc.s, t2 = acc.s2;
+    if (gw > 0 && g == 0) {
+      red[(gw - 1) * 2 * BK + key] = t1;
+      if constexpr (EPI == kColSumSq) red[(gw - 1) * 2 * BK + BK + key] = t2;
     }
     __syncthreads();
-    if (gw == 0 && g == 0) {
+    if (gw == 0 && g == 0 && kj < p.Sk) {
 #pragma unroll
-      for (int kb = 0; kb < KPW; ++kb) {
-        const int key = 32 * (KPW * wi + kb) + r, kjb = kj + 32 * kb;
-        if (kjb < p.Sk) {
-          p.colsum[(int64_t)bh * p.Sk + kjb] = acc[kb].s + red[key];
-          if constexpr (EPI == kColSumSq) p.colsum2[(int64_t)bh * p.Sk + kjb] = acc[kb].s2 + red[BK + key];
-        }
+      for (int i = 0; i < NG - 1; ++i) {
+        t1 += red[i * 2 * BK + key];
+        if constexpr (EPI == kColSumSq) t2 += red[i * 2 * BK + BK + key];
+      }
+      if constexpr (EPI == kColAnyGe) {
+        p.any_out[(int64_t)bh * p.Sk + kj] = t1 != 0.0f;
+      } else {
+        p.colsum[(int64_t)bh * p.Sk + kj] = t1;
+        if constexpr (EPI == kColSumSq) p.colsum2[(int64_t)bh * p.Sk + kj] = t2;
       }
     }
   }
 }
 
 template <typename T, int D, bool MASK, bool SOFTCAP, int REFROUND, int EPI>
-void launch_colsum(const AttnParams& p, hipStream_t st) {
+void launch_colsum(AttnParams p, hipStream_t st) {
+  p.n_tiles = (p.Sk + kCBK - 1) / kCBK;
   const unsigned grid = (unsigned)p.n_tiles * p.B * p.Hq;
   hipLaunchKernelGGL((attn_colsum_kernel<T, D, MASK, SOFTCAP, REFROUND, EPI>), dim3(grid), dim3(kThreads), 0, st, p);
 }
 
-// head_dim 128 column sums (measured on MI355X, config 4): 8 waves x 32 keys, 128-row query tiles, 2 stages.
-// DGG_COL_PIPE (default 1): the sum epilogues (H2O / SnapKV, RoCo) run the software-pipelined 3-stage form.
-#ifndef DGG_COL_PIPE
-#define DGG_COL_PIPE 1
-#endif
-// DGG_COL_KPW: 32-key blocks per wave in the pipelined form (2; 1: 8 waves x 32 keys over 128-row tiles).
-#ifndef DGG_COL_KPW
-#define DGG_COL_KPW 2
-#endif
-constexpr int kC128NW = 8, kC128BQ = 128, kC128NS = 2;
-constexpr int kC128BK = 32 * kC128NW;  // keys per workgroup (head_dim 128)
+template <typename T, int NG, int OCC, bool MASK, bool SOFTCAP, int REFROUND, int EPI>
+void launch_colsum_d128_form(AttnParams p, hipStream_t st) {
+  constexpr int NW = 8, BQ = 128, BK = 32 * NW / NG;
+  p.n_tiles = (p.Sk + BK - 1) / BK;
+  const unsigned grid = (unsigned)p.n_tiles * p.B * p.Hq;
+  if (p.lse_base2)
+    hipLaunchKernelGGL((attn_colsum_d128_kernel<T, NW, NG, BQ, OCC, MASK, SOFTCAP, REFROUND, true, EPI>), dim3(grid),
+                       dim3(64 * NW), 0, st, p);
+  else
+    hipLaunchKernelGGL((attn_colsum_d128_kernel<T, NW, NG, BQ, OCC, MASK, SOFTCAP, REFROUND, false, EPI>), dim3(grid),
+                       dim3(64 * NW), 0, st, p);
+}
 
+// head_dim 128 column passes: 8 waves, 128-row query tiles; 64 keys per workgroup in four row groups (NG 4) or 128 in
+// two (NG 2). What counts is four waves per SIMD: each score costs ~6 vector instructions and one exponential against
+// 1/32 of an MFMA, so waves at different points of their tiles fill the pipes better than any fixed order within one
+// (fp16 reference-rounded sums, H=32, causal, S=4096: 92.3 us; 95.7 us for two waves per SIMD running the products of
+// one tile under the exponentials of the previous, 256 keys per workgroup; 105 us for NG 2 at two waves per SIMD).
+// * Sums: NG 4 up to 768 workgroups of 64 keys (S=1000: 12.6 us, NG 2 17.0; S=1536 19.9 / 21.5), NG 2 beyond, where
+//   the chip is full and each query tile is read by half as many workgroups (2 x 1024: 17.3, NG 4 19.0).
+// * Corm: NG 4 always (S=4096 44.3 us, NG 2 50.0 at its best, two waves per SIMD: its thresholds do not fit the
+//   registers of four); the reference-rounded soft-cap likewise.
+// * KeyFormer: NG 4 up to the same size (S=1000 19.7 us, NG 2 27.8); beyond, NG 2 at two waves per SIMD, whose rows of
+//   exp_rand are read 512 bytes at a time (S=2048 64.9 us, NG 4 76.9; equal at S=4096).
 template <typename T, bool MASK, bool SOFTCAP, int REFROUND, int EPI>
 void launch_colsum_d128(const AttnParams& p, hipStream_t st) {
-  const unsigned grid = (unsigned)p.n_tiles * p.B * p.Hq;
-  // (the reference-rounded soft-cap's score chain is too long for a fixed-order step: it keeps the plain form)
-  constexpr bool PIPE = DGG_COL_PIPE && (EPI == kColSum || EPI == kColSumSq) && !(SOFTCAP && REFROUND);
-  constexpr int NS = PIPE ? 3 : kC128NS;
-  // The pipelined form: 64 keys per wave, the 8 waves in two row groups of 4 (each group takes 64 rows of every
-  // 128-row query tile); the same 256 keys per workgroup.
-  constexpr int KPW = PIPE ? DGG_COL_KPW : 1;
-  constexpr int NW = kC128NW, BQ = kC128BQ;
-  static_assert(32 * NW == kC128BK, "keys per workgroup");
-  if (p.lse_base2)
-    hipLaunchKernelGGL((attn_colsum_d128_kernel<T, NW, KPW, BQ, NS, MASK, SOFTCAP, REFROUND, true, EPI>),
-                       dim3(grid), dim3(64 * NW), 0, st, p);
-  else
-    hipLaunchKernelGGL((attn_colsum_d128_kernel<T, NW, KPW, BQ, NS, MASK, SOFTCAP, REFROUND, false, EPI>),
-                       dim3(grid), dim3(64 * NW), 0, st, p);
+  const bool small = (int64_t)((p.Sk + 63) / 64) * p.B * p.Hq <= 768;
+  constexpr bool NG4 = EPI == kColAnyGe || (SOFTCAP && REFROUND);
+  if (NG4 || small) return launch_colsum_d128_form<T, 4, 4, MASK, SOFTCAP, REFROUND, EPI>(p, st);
+  if constexpr (!NG4)
+    launch_colsum_d128_form<T, 2, EPI == kColKF ? 2 : 4, MASK, SOFTCAP, REFROUND, EPI>(p, st);
 }
 
 template <typename T, int D, bool MASK, bool SOFTCAP, int REFROUND, int EPI>
@@ -926,6 +1036,13 @@ void pick_col(const AttnParams& p, bool ref, int epi, hipStream_t st) {
 template <typename T, int D, bool MASK, int REFROUND>
 void launch_kf_rowlse(const AttnParams& p, bool vec, hipStream_t st) {
   const unsigned grid = (unsigned)p.n_tiles * p.B * p.Hq;
+  if constexpr (D == 128) {
+    // exp_rand as whole 16-byte chunks: aligned rows and a key count that ends on a chunk
+    if (vec && p.Sk % 4 == 0) {
+      hipLaunchKernelGGL((attn_kf_rowlse_dma_kernel<T, MASK, REFROUND>), dim3(grid), dim3(512), 0, st, p);
+      return;
+    }
+  }
   if (vec) hipLaunchKernelGGL((attn_kf_rowlse_kernel<T, D, MASK, REFROUND, true>), dim3(grid), dim3(kThreads), 0, st, p);
   else hipLaunchKernelGGL((attn_kf_rowlse_kernel<T, D, MASK, REFROUND, false>), dim3(grid), dim3(kThreads), 0, st, p);
 }
@@ -1135,8 +1252,6 @@ int colscore(const char* op, const void* q, const void* k, const float* lse, int
     p.n_tiles = (int)((Sk + f32_rows_per_tile() - 1) / f32_rows_per_tile());
     launch_attn_f32_col(p, (int)D, epi, st);
   } else {
-    const int64_t bk = D == 128 ? kC128BK : kCBK;
-    p.n_tiles = (int)((Sk + bk - 1) / bk);
     const bool ref = (flags & DGG_ATTN_REF_ROUNDING) != 0;
     if (dtype == DGG_BF16) {
       if (D == 64) pick_col<BF16, 64>(p, ref, epi, st);
@@ -1233,8 +1348,6 @@ extern "C" int dgg_attn_kf_colsum(const void* q, const void* k, const float* exp
   p.q_sb = strides[0]; p.q_ss = strides[1]; p.q_sh = strides[2];
   p.k_sb = strides[3]; p.k_ss = strides[4]; p.k_sh = strides[5];
   if (Sq > 0) set_exp_rand(p, exp_rand, er_strides, tau);
-  const int64_t bk = D == 128 ? kC128BK : kCBK;
-  p.n_tiles = (int)((Sk + bk - 1) / bk);
   const bool ref = (flags & DGG_ATTN_REF_ROUNDING) != 0;
   hipStream_t st = dgg::as_stream(stream);
   if (dtype == DGG_BF16) {

@@ -134,12 +134,6 @@ struct ColAcc {
       if constexpr (EPI == kColSumSq) s2 = fmaf(pe, pe, s2);
     }
   }
-  // Ties the sums so far to this point of the program (a fixed-order schedule would otherwise see its additions
-  // sunk past later code that does not use them).
-  __device__ __forceinline__ void pin() {
-    if constexpr (EPI != kColAnyGe) asm volatile("" : "+v"(s));
-    if constexpr (EPI == kColSumSq) asm volatile("" : "+v"(s2));
-  }
   // Combines the two lane halves (rows 4g..) and stores column kj of (batch, head) bh.
   __device__ __forceinline__ void store(const AttnParams& p, int bh, int kj, int g) {
     if constexpr (EPI == kColAnyGe) {
@@ -169,17 +163,25 @@ __device__ __forceinline__ f16x2 ref_scores_f16(float a, float b, const AttnPara
 
 // Maps blockIdx.x to (tile, batch*head). Longest tiles first; when the (batch, head) count divides by 8,
 // each XCD gets a contiguous group of heads so their K/V are shared through that XCD's L2.
+// PAIR, for kernels of which a CU holds two workgroups: a launch of between one and two per CU is resident at once, the
+// workgroups after the first 256 joining them in order. Taking those from the short end gives every CU a long and a
+// short tile, not the i-th longest and the (i + 256)-th.
+template <bool PAIR = false>
 __device__ __forceinline__ void map_block(int n_tiles, int bh_count, bool reverse, int& tile, int& bh) {
   const int bid = blockIdx.x;
+  const bool pair = PAIR && n_tiles * bh_count > 256 && n_tiles * bh_count <= 512;
   int t_major, bh_minor;
   if ((bh_count & 7) == 0) {
     const int hpx = bh_count >> 3;
-    const int xcd = bid & 7, local = bid >> 3;
+    const int xcd = bid & 7;
+    int local = bid >> 3;
+    if (pair && local >= 32) local = n_tiles * hpx - 1 - (local - 32);
     t_major = local / hpx;
     bh_minor = xcd * hpx + (local - t_major * hpx);
   } else {
-    t_major = bid / bh_count;
-    bh_minor = bid - t_major * bh_count;
+    const int i = pair && bid >= 256 ? n_tiles * bh_count - 1 - (bid - 256) : bid;
+    t_major = i / bh_count;
+    bh_minor = i - t_major * bh_count;
   }
   tile = reverse ? n_tiles - 1 - t_major : t_major;
   bh = bh_minor;

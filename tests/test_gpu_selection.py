@@ -314,3 +314,25 @@ def test_selection_full_size_heads(gpu):
     _, kf = A.keyformer_attention(qg, kg, vg, er.to(gpu))
     assert_close(kf.cpu(), ref_kf, 1e-6, 1e-3, "kf_score full")
     np.testing.assert_array_equal(A.topk_indices(kf, 256).cpu().numpy(), osel.topk_indices(ref_kf.numpy(), 256))
+
+
+@pytest.mark.parametrize("S", [448, 577])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_column_forms_agree(gpu, S, dtype):
+    """The column passes of large launches (128 keys per workgroup in two row groups, from more than 768 workgroups of 64
+    keys) against those of small ones (64 keys, four groups), which the oracle tests cover: 112 heads in one call and
+    three of them in a call of their own. The same fp32 terms in another order: 577 of them, each sum within
+    577 * 2^-24 = 3.4e-5 of exact in the worst case (twice that for the two together)."""
+    H, hs = 112, [0, 50, 111]
+    q, k, v = (t.to(gpu) for t in _qkv(S, H, 128, S, dtype=dtype, sinks=4))
+    er = 1.0 + torch.randn(1, H, S, S, generator=torch.Generator(device=gpu).manual_seed(S), device=gpu).abs()
+    some = [t[:, :, hs].contiguous() for t in (q, k, v)]
+    for ref_rounding in (True, False):
+        big = A.roco_attention(q, k, v, ref_rounding=ref_rounding)
+        few = A.roco_attention(*some, ref_rounding=ref_rounding)
+        # the forward picks its form by the launch's size too: its row lse may differ in the last bits
+        for b, f, what in zip(big[1:], few[1:], ("sum", "sum of squares")):
+            assert_close(b[:, hs].cpu(), f.cpu(), 1e-7, 7e-5, f"roco {what} S{S} {dtype} ref={ref_rounding}")
+        big = A.keyformer_attention(q, k, v, er, ref_rounding=ref_rounding)[1]
+        few = A.keyformer_attention(*some, er[:, hs].contiguous(), ref_rounding=ref_rounding)[1]
+        assert_close(big[:, hs].cpu(), few.cpu(), 1e-7, 7e-5, f"keyformer S{S} {dtype} ref={ref_rounding}")
