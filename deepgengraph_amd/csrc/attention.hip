@@ -1160,7 +1160,6 @@ int prefill_impl(const char* op, const void* q, const void* k, const void* v, vo
   hipStream_t st = dgg::as_stream(stream);
   // Sk == 0 still launches and writes o = 0 (the reference's P.V over an empty key axis) and lse = -inf.
   if (dtype == DGG_F32) {  // fp32 has no 16-bit rounding point: reference rounding changes nothing
-    p.n_tiles = (int)((Sq + f32_rows_per_tile() - 1) / f32_rows_per_tile());
     launch_attn_f32_fwd(p, (int)D, st);
     return dgg::check_launch(op);
   }

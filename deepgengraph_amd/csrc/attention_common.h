@@ -354,7 +354,8 @@ void launch_attn_d256_pipe(const AttnParams& p, bool bf16, hipStream_t st);
 void launch_attn_fwd_f16(const AttnParams& p, int D, bool ref, hipStream_t st);
 void launch_attn_fwd_bf16(const AttnParams& p, int D, bool ref, hipStream_t st);
 
-// fp32 inputs (attention_f32.hip): the forward and the column-score pass, rows per workgroup tile of both.
+// fp32 inputs (attention_f32.hip): the forward (which sets its own tile count) and the column-score pass, keys per
+// workgroup of the latter.
 int f32_rows_per_tile();
 void launch_attn_f32_fwd(const AttnParams& p, int D, hipStream_t st);
 void launch_attn_f32_col(const AttnParams& p, int D, int epi, hipStream_t st);

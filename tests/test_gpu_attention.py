@@ -219,6 +219,22 @@ def test_prefill_fp32_matches_oracle(gpu, B, Sq, Sk, Hq, Hkv, D, causal, softcap
     assert_close(lse.cpu()[fin], ref_lse[fin], 1e-5, 1e-6, what + " lse")
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("Sq,Sk,causal,window", [(1, 1, True, 0), (15, 17, True, 0), (16, 64, False, 0), (17, 5, False, 0),
+                                                 (33, 16, True, 0), (49, 80, True, 9), (31, 100, False, 30)])
+def test_prefill_fp32_block_edges(gpu, D, Sq, Sk, causal, window):
+    """Edges of the fp32 forward's 16-row and 16-key blocks and of its four-way key split (waves with no block, with
+    masked blocks only, rows that see no key): 1e-5 as the fp32 cases above, some 20x the rounding of these sums."""
+    q, k, v = _qkv(2, Sq, Sk, 4, 2, D, torch.float32, seed=Sq + Sk + D)
+    ref, ref_lse = oa.attention(q, k, v, causal=causal, window=window or None, return_lse=True)
+    out, lse = A.attention(q.to(gpu), k.to(gpu), v.to(gpu), causal=causal, window=window, return_lse=True)
+    what = f"fp32 Sq{Sq} Sk{Sk} D{D} causal={causal} win={window}"
+    assert_close(out.cpu(), ref, 1e-5, 1e-5, what)
+    fin = torch.isfinite(ref_lse)
+    assert torch.equal(torch.isfinite(lse.cpu()), fin), what + " lse -inf pattern"
+    assert_close(lse.cpu()[fin], ref_lse[fin], 1e-5, 1e-5, what + " lse")
+
+
 def test_config1_fp32_on_gpu(gpu):
     # config 1 (fp32, B=1, H=8, S=512, D=64) through the C ABI: O and LSE against the oracle, and through the
     # drop-in compile(Attn) callable
