@@ -59,16 +59,15 @@ def _splitkv_shaped(Sq: int, Sk: int, Hq: int, Hkv: int, ref_rounding: bool, dty
 
 
 def splitkv_splits(B: int, Sq: int, Hq: int, Hkv: int, span: int) -> int:
-    """Key slices for a split-KV call over `span` keys: about 1024 workgroups over the chip, each slice at least 512
-    keys and at least 32 keys per row it serves, so that the partials written and merged stay a few percent of the
-    K / V bytes read. (Measured on MI355X at 32K keys: q_len 1-16 over 32 heads ran best with 16-32 slices, 5.0-5.2
-    TB/s, against 4.2-4.7 TB/s with 256; q_len 64 with 16.)"""
+    """Key slices for a split-KV call over `span` keys: up to 512 workgroups (1024 for at most 8 rows per KV head, whose
+    partials are small), each slice at least 32 keys and 8 per row it serves, and at most 64 slices below 16K keys, whose
+    merge would take longer than the keys. The library's own rule for grouped-query decode (splitkv_useful_splits in
+    csrc/splitkv.hip, with the measurements)."""
     rows = (Hq // Hkv) * Sq
-    rpw = 32 if rows <= 32 else 64
-    groups = B * Hkv * (-(-rows // rpw))
-    want = -(-1024 // max(1, groups))
-    min_keys = max(512, 32 * min(rows, rpw))
-    return int(max(1, min(1024, want, -(-span // min_keys))))
+    groups = max(1, B * Hkv * (-(-rows // (32 if rows <= 32 else 64))))
+    want = -(-(1024 if rows <= 8 else 512) // groups)
+    min_keys = max(32, 8 * min(rows, 32))
+    return int(max(1, min(want, 64 if span < 16384 else 1024, -(-span // min_keys))))
 
 
 def decode_splits(B: int, Hq: int, L: int) -> int:

@@ -38,6 +38,9 @@ int splitkv_launch(const char* op, const void* q, const void* k, const void* v, 
                    const int64_t* strides, int64_t splits, float scale, float softcap, int64_t window, uint32_t flags,
                    int dtype, void* stream, int (*resolve_ws)(const char* op, void* stream, void** ws));
 
+// Number of key slices of a split-KV call over `span` keys beyond which more slices only add partials (splitkv.hip).
+int64_t splitkv_useful_splits(int64_t B, int64_t Sq, int64_t Hq, int64_t Hkv, int64_t span);
+
 }  // namespace dgg
 
 #define DGG_REQUIRE(cond, code, ...)            \

@@ -138,18 +138,23 @@ __global__ void __launch_bounds__(kDecThreads) decode_partial_kernel(DecodeParam
     for (int i = 0; i < GROUPS; ++i) M = fmaxf(M, sm[i]);
     const float Mu = M == -INFINITY ? 0.f : M;
     const int64_t pidx = ((int64_t)b * p.Hq + h) * p.splits + split;
+    float L = 0.f;
+#pragma unroll
+    for (int i = 0; i < GROUPS; ++i) L += fast_exp2(sm[i] - Mu) * sl[i];
     for (int d = tid; d < D; d += kDecThreads) {
       float od = 0.f;
 #pragma unroll
       for (int i = 0; i < GROUPS; ++i) od += fast_exp2(sm[i] - Mu) * so[i][d];
-      p.part_o[pidx * D + d] = od;
+      if (p.splits == 1) static_cast<S*>(p.o)[b * p.o_sb + h * p.o_sh + d] = to_s<S>(od / L);  // nothing to merge
+      else p.part_o[pidx * D + d] = od;
     }
     if (tid == 0) {
-      float L = 0.f;
-#pragma unroll
-      for (int i = 0; i < GROUPS; ++i) L += fast_exp2(sm[i] - Mu) * sl[i];
-      p.part_ml[pidx * 2 + 0] = M;
-      p.part_ml[pidx * 2 + 1] = L;
+      if (p.splits == 1) {
+        if (p.lse != nullptr) p.lse[(int64_t)b * p.Hq + h] = (M == -INFINITY ? -INFINITY : M + fast_log2(L)) * kLn2;
+      } else {
+        p.part_ml[pidx * 2 + 0] = M;
+        p.part_ml[pidx * 2 + 1] = L;
+      }
     }
     if (nsplit >= s_end) break;
     __syncthreads();  // every lane group has read sm / sl / so before the next split's merge rewrites them
@@ -189,10 +194,21 @@ __global__ void __launch_bounds__(256) decode_merge_kernel(DecodeParams p) {
   }
 }
 
+// Splits a call runs with, of the `splits` it was given (its workspace is sized for those): enough for ~512 workgroups,
+// or up to 8 of at least 4,096 keys, and at least 128 keys each (one unrolled block of the partial kernel; with fewer
+// the block re-reads its last key). More splits only add partials and their merge. Measured on MI355X, D=128, bf16, at 64
+// splits and at the number this picks: B=64, H=32, L=128 855 -> 28 us (1); L=2048 895 -> 314 (1); B=16, L=1024 238 -> 45
+// (1); B=1, L=4096 35.8 -> 18.5 (16); B=64, L=8192 1445 -> 1229 (2).
+int64_t decode_useful_splits(int64_t splits, int64_t BH, int64_t L) {
+  const int64_t want = std::max((512 + BH - 1) / BH, std::min<int64_t>(8, (L + 4095) / 4096));
+  return std::max<int64_t>(1, std::min({splits, want, (L + 127) / 128}));
+}
+
 template <typename T, int D>
 void launch_decode(const DecodeParams& p, hipStream_t st) {
   hipLaunchKernelGGL((decode_partial_kernel<T, D>), dim3((p.splits + kSplitsPerWg - 1) / kSplitsPerWg, p.Hq, p.B), dim3(kDecThreads), 0, st, p);
-  hipLaunchKernelGGL((decode_merge_kernel<T, D>), dim3(p.Hq, p.B), dim3(D < 256 ? 128 : 256), 0, st, p);
+  if (p.splits > 1)
+    hipLaunchKernelGGL((decode_merge_kernel<T, D>), dim3(p.Hq, p.B), dim3(D < 256 ? 128 : 256), 0, st, p);
 }
 
 }  // namespace
@@ -241,6 +257,7 @@ int decode_launch(const char* op, const void* q, const void* k, const void* v, v
     // strides {b, l, h}; the partials have the same size.
     const int64_t st12[12] = {strides[0], 0,          strides[1], strides[2], strides[4], strides[3],
                               strides[5], strides[7], strides[6], strides[8], 0,          strides[9]};
+    splits = std::min(splits, dgg::splitkv_useful_splits(B, 1, Hq, Hkv, L));
     return dgg::splitkv_launch(op, q, k, v, o, lse, workspace, workspace_bytes, B, 1, L, Hq, Hkv, D, st12, splits,
                                scale, 0.f, 0, 0u, dtype, stream, resolve_ws);
   }
@@ -257,7 +274,7 @@ int decode_launch(const char* op, const void* q, const void* k, const void* v, v
   p.o = o;
   p.lse = lse;
   p.part_o = static_cast<float*>(workspace);
-  p.part_ml = p.part_o + B * Hq * splits * D;
+  p.part_ml = p.part_o + B * Hq * splits * D;  // (of the splits given)
   p.q_sb = strides[0]; p.q_sh = strides[1];
   p.k_sb = strides[2]; p.k_sh = strides[3]; p.k_sl = strides[4];
   p.v_sb = strides[5]; p.v_sh = strides[6]; p.v_sl = strides[7];
@@ -267,8 +284,9 @@ int decode_launch(const char* op, const void* q, const void* k, const void* v, v
   p.Hkv = (int)Hkv;
   p.group = (int)(Hq / Hkv);
   p.L = (int)L;
-  p.splits = (int)splits;
+  splits = decode_useful_splits(splits, B * Hq, L);
   p.chunk = (int)((L + splits - 1) / splits);
+  p.splits = (int)((L + p.chunk - 1) / p.chunk);
   p.c = scale * kLog2e;
   hipStream_t st = dgg::as_stream(stream);
   if (dtype == DGG_BF16) {

@@ -323,6 +323,23 @@ void pick_splitkv(const SplitParams& sp, int nw, hipStream_t st) {
 
 namespace dgg {
 
+// (attention.py's splitkv_splits is the same rule, for calls that size their own workspace.)
+// A workgroup serves up to 32 rows of a KV head with one wave, 64 with two; a slice's latency is one tile of 32 keys after
+// another, so small calls want many short slices, as long as the partials (rows * (D + 2) floats a slice) stay small
+// against the keys and the merge short. Measured on MI355X, D=128, bf16, us at the number picked (and at a half and twice):
+// B=1, 1 row, 32 / 8 heads: 4,001 keys 64: 9.7 (32: 10.8, 8: 22.2); 1,024 keys 32: 7.8 (16: 9.0); 32,768 keys 128: 27.2
+// (64: 29.5, 256: 28.6). B=8, 4,001 keys 16: 28.2 (8: 29.4, 32: 29.7). 16 rows, 32 heads: 8,192 keys 16: 30.8 (8: 39.8,
+// 32: 31.3); 2,048 keys 16: 14.3 (8: 15.9, 32: 16.4). 16 rows, 32 / 8 heads: 8,192 keys 32: 19.1 (16: 23.2, 64: 21.9).
+// 64 rows, 32 heads: 2,048 keys 8: 19.6 (4: 23.7, 16: 22.0).
+int64_t splitkv_useful_splits(int64_t B, int64_t Sq, int64_t Hq, int64_t Hkv, int64_t span) {
+  const int64_t rows = std::max<int64_t>(1, Hq / Hkv * Sq), rpw = rows <= 32 ? 32 : 64;
+  const int64_t groups = std::max<int64_t>(1, B * Hkv * ((rows + rpw - 1) / rpw));
+  const int64_t want = ((rows <= 8 ? 1024 : 512) + groups - 1) / groups;
+  const int64_t min_keys = std::max<int64_t>(32, 8 * std::min<int64_t>(rows, 32));
+  const int64_t cap = span < 16384 ? 64 : 1024;
+  return std::max<int64_t>(1, std::min({want, cap, (span + min_keys - 1) / min_keys}));
+}
+
 // Shared body of dgg_attn_splitkv and of dgg_attn_decode / dgg_attn_decode_noalloc for grouped query heads (declared
 // in common.h).
 int splitkv_launch(const char* op, const void* q, const void* k, const void* v, void* o, float* lse, void* workspace,
@@ -374,9 +391,9 @@ int splitkv_launch(const char* op, const void* q, const void* k, const void* v, 
   chunk = (chunk + kSkBN - 1) / kSkBN * kSkBN;
   sp.k_first = (int)k_first;
   sp.chunk = (int)chunk;
-  sp.splits = (int)splits;
   sp.part_o = static_cast<float*>(workspace);
   sp.part_ml = sp.part_o + B * Hq * Sq * splits * D;
+  sp.splits = (int)((span + chunk - 1) / chunk);  // slices that hold a key
   hipStream_t st = dgg::as_stream(stream);
   if (dtype == DGG_BF16) {
     if (D == 64) pick_splitkv<BF16, 64>(sp, nw, st);

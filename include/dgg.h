@@ -257,7 +257,8 @@ int dgg_roco_select_ws(const float* score, const float* sq_score, int64_t rows, 
  * strides: 10 int64 = q{b,h}, k{b,h,l}, v{b,h,l}, o{b,h}.
  * workspace: fp32 scratch of dgg_attn_decode_workspace_bytes(B, Hq, D, splits) bytes, 16B aligned:
  * per (b, h, split) the unnormalised partial output, its max and its sum.
- * lse (optional): fp32 [B, Hq], natural log. splits in [1, 1024]; L >= 1. */
+ * lse (optional): fp32 [B, Hq], natural log. splits in [1, 1024]: the most splits the call runs with (it takes fewer
+ * where more would only add partials); L >= 1. */
 int64_t dgg_attn_decode_workspace_bytes(int64_t B, int64_t Hq, int64_t D, int64_t splits);
 int dgg_attn_decode(const void* q, const void* k, const void* v, void* o, float* lse, void* workspace,
                     int64_t workspace_bytes, int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t D,
