@@ -114,10 +114,9 @@ def load() -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
     """Calls a status-returning entry point; raises RuntimeError with dgg_last_error() on failure."""
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    rc = getattr(_lib or load(), name)(*args)
     if rc != 0:
-        msg = lib.dgg_last_error().decode(errors="replace")
+        msg = load().dgg_last_error().decode(errors="replace")
         raise RuntimeError(f"{name} failed ({rc}): {msg}")
 
 
@@ -128,16 +127,32 @@ def dtype_code(t: torch.dtype) -> int:
         raise RuntimeError(f"unsupported dtype {t} (expected float32, float16 or bfloat16)") from None
 
 
+# The small calls of this framework take the GPU 5-15 us, so what the host does per call is most of their time. The
+# helpers below are therefore the plain forms: an address as an int (the c_void_p argument types take it as it is), the
+# raw stream without a Stream object, an array type looked up once.
 def ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def stream_handle(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def stream_handle(device: torch.device):
+    """The current stream of the device, as the address the library takes (0 / None: the null stream)."""
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
+
+
+_I64_ARRAY = {}
 
 
 def int64_array(vals) -> ctypes.Array:
-    return (ctypes.c_int64 * len(vals))(*[int(v) for v in vals])
+    n = len(vals)
+    cls = _I64_ARRAY.get(n)
+    if cls is None:
+        cls = _I64_ARRAY[n] = ctypes.c_int64 * n
+    return cls(*vals)
 
 
 def require_gpu(*tensors: torch.Tensor) -> torch.device:

@@ -13,10 +13,16 @@ from . import _lib
 
 
 def _check_bshd(name: str, t: torch.Tensor):
-    if t.dim() != 4:
+    st = t.stride()
+    if len(st) != 4:
         raise RuntimeError(f"{name}: expected [B, S, H, D], got shape {tuple(t.shape)}")
-    if t.stride(-1) != 1:
-        raise RuntimeError(f"{name}: head dimension must be contiguous (stride {t.stride(-1)})")
+    if st[3] != 1:
+        raise RuntimeError(f"{name}: head dimension must be contiguous (stride {st[3]})")
+
+
+def _strides3(*tensors: torch.Tensor):
+    """The batch, sequence and head strides of [B, S, H, D] tensors, one after the other, as the library takes them."""
+    return _lib.int64_array([x for t in tensors for x in t.stride()[:3]])
 
 
 def _check_qk(name: str, q: torch.Tensor, k: torch.Tensor):
@@ -155,11 +161,12 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool
     kernel by its row of this table (rotary_cos_sin of the rows' positions, [B * Sq, 128], batch-major), as
     rotary_embedding_online would have rotated it in place (models/attn.py:41); q is not modified."""
     dev = _lib.require_gpu(q, k, v, out, rope_cos_sin)
-    for name, t in (("q", q), ("k", k), ("v", v)):
-        _check_bshd(name, t)
+    _check_bshd("q", q)
+    _check_bshd("k", k)
+    _check_bshd("v", v)
     B, Sq, Hq, D = q.shape
-    Sk, Hkv = k.shape[1], k.shape[2]
-    if k.shape[0] != B or v.shape != k.shape or k.shape[3] != D:
+    Bk, Sk, Hkv, Dk = k.shape
+    if Bk != B or v.shape != k.shape or Dk != D:
         raise RuntimeError(f"attention: incompatible shapes q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)}")
     if not (q.dtype == k.dtype == v.dtype):
         raise RuntimeError("attention: q, k, v dtypes differ")
@@ -178,7 +185,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool
             raise RuntimeError(f"attention: rope_cos_sin must be a contiguous fp32 [{B * Sq}, {D}] tensor")
         flags = ((_lib.ATTN_CAUSAL if causal else 0) | (_lib.ATTN_REF_ROUNDING if ref_rounding else 0)
                  | (_lib.ATTN_LSE_BASE2 if lse_base2 else 0))
-        strides = _lib.int64_array([*q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *out.stride()[:3]])
+        strides = _strides3(q, k, v, out)
         _lib.call("dgg_attn_prefill_rope", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), _lib.ptr(lse), B, Sq,
                   Sk, Hq, Hkv, D, strides, scale, float(softcap or 0.0), int(window or 0), flags,
                   _lib.dtype_code(q.dtype), _lib.ptr(rope_cos_sin), _lib.stream_handle(dev))
@@ -202,7 +209,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool
         return (out, lse) if return_lse else out
     flags = ((_lib.ATTN_CAUSAL if causal else 0) | (_lib.ATTN_REF_ROUNDING if ref_rounding else 0)
              | (_lib.ATTN_LSE_BASE2 if lse_base2 else 0))
-    strides = _lib.int64_array([*q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *out.stride()[:3]])
+    strides = _strides3(q, k, v, out)
     _lib.call("dgg_attn_prefill", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), _lib.ptr(lse), B, Sq, Sk,
               Hq, Hkv, D, strides, scale, float(softcap or 0.0), int(window or 0), flags, _lib.dtype_code(q.dtype),
               _lib.stream_handle(dev))
@@ -215,12 +222,12 @@ def _splitkv(q, k, v, out, lse, causal, softcap, window, scale, lse_base2, split
     if splits is None:
         first = max(0, Sk - Sq - window + 1) if window else 0
         splits = splitkv_splits(B, Sq, Hq, Hkv, Sk - first)
-    need = int(_lib.load().dgg_attn_splitkv_workspace_bytes(B, Sq, Hq, D, splits))
-    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=q.device)
+    # dgg_attn_splitkv_workspace_bytes: an unnormalised output row, its maximum and its sum per row and slice
+    ws = torch.empty(max(B * Sq * Hq * splits * (D + 2), 4), dtype=torch.float32, device=dev)
     flags = (_lib.ATTN_CAUSAL if causal else 0) | (_lib.ATTN_LSE_BASE2 if lse_base2 else 0)
-    strides = _lib.int64_array([*q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *out.stride()[:3]])
+    strides = _strides3(q, k, v, out)
     _lib.call("dgg_attn_splitkv", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), _lib.ptr(lse), _lib.ptr(ws),
-              ws.numel(), B, Sq, Sk, Hq, Hkv, D, strides, int(splits), float(scale), float(softcap or 0.0),
+              4 * ws.numel(), B, Sq, Sk, Hq, Hkv, D, strides, int(splits), float(scale), float(softcap or 0.0),
               int(window or 0), flags, _lib.dtype_code(q.dtype), _lib.stream_handle(dev))
 
 
@@ -271,7 +278,7 @@ def attention_colsum(q: torch.Tensor, k: torch.Tensor, lse: torch.Tensor, *, cau
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
     flags = ((_lib.ATTN_CAUSAL if causal else 0) | (_lib.ATTN_REF_ROUNDING if ref_rounding else 0)
              | (_lib.ATTN_LSE_BASE2 if lse_base2 else 0))
-    strides = _lib.int64_array([*q.stride()[:3], *k.stride()[:3]])
+    strides = _strides3(q, k)
     _lib.call("dgg_attn_colsum", _lib.ptr(q), _lib.ptr(k), _lib.ptr(lse), _lib.ptr(colsum), B, Sq, Sk, Hq, Hkv, D,
               strides, scale, float(softcap or 0.0), int(window or 0), flags, _lib.dtype_code(q.dtype),
               _lib.stream_handle(dev))
@@ -320,7 +327,7 @@ def attention_colscore(q: torch.Tensor, k: torch.Tensor, lse: torch.Tensor, *, e
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
     flags = ((_lib.ATTN_CAUSAL if causal else 0) | (_lib.ATTN_REF_ROUNDING if ref_rounding else 0)
              | (_lib.ATTN_LSE_BASE2 if lse_base2 else 0))
-    strides = _lib.int64_array([*q.stride()[:3], *k.stride()[:3]])
+    strides = _strides3(q, k)
     _lib.call("dgg_attn_colscore", _lib.ptr(q), _lib.ptr(k), _lib.ptr(lse), int(epilogue), _lib.ptr(out0),
               _lib.ptr(out1), _lib.ptr(anyo), _lib.ptr(thr), thr_rs, B, Sq, Sk, Hq, Hkv, D, strides, scale, 0.0,
               int(window or 0), flags, _lib.dtype_code(q.dtype), _lib.stream_handle(dev))
@@ -395,7 +402,7 @@ def keyformer_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, exp_r
     out = attention(q, k, v, causal=True, ref_rounding=ref_rounding)
     scale = 1.0 / math.sqrt(D)
     flags = _lib.ATTN_CAUSAL | (_lib.ATTN_REF_ROUNDING if ref_rounding else 0)
-    strides = _lib.int64_array([*q.stride()[:3], *k.stride()[:3]])
+    strides = _strides3(q, k)
     er_strides = _lib.int64_array(list(exp_rand.stride()[:3]))
     lse2 = torch.empty(B, H, Sq, dtype=torch.float32, device=q.device)
     _lib.call("dgg_attn_kf_rowlse", _lib.ptr(q), _lib.ptr(k), _lib.ptr(exp_rand), er_strides, _lib.ptr(lse2), B, Sq,

@@ -17,8 +17,11 @@ def _rows(t: torch.Tensor, what: str):
     if t.dim() == 0:
         raise RuntimeError(f"{what}: expected at least one dimension")
     n = t.shape[-1]
-    if t.numel() == 0:
+    numel = t.numel()
+    if numel == 0:
         return 0, max(n, 1)
+    if t.is_contiguous():
+        return numel // n, n
     if t.stride(-1) != 1 and n > 1:
         raise RuntimeError(f"{what}: innermost dimension must be contiguous (stride {t.stride(-1)})")
     if t.dim() == 1:
