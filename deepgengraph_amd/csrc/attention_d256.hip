@@ -46,6 +46,8 @@ attn_fwd_d256_pipe_kernel(AttnParams p) {
   constexpr int GPW = (BN / 4) / NW;          // 4-row groups of a tile copied by each wave
   constexpr int DMA_PER_TILE = GPW * IPG;     // direct loads per wave per K (or V) tile
   constexpr int NMB = BN / 32;                // 32-key blocks per tile
+  constexpr int QSLOT_B = 8 * GROUP_B;        // 32 rows of Q (at the start) or O (at the end)
+  static_assert(2 * QSLOT_B == TILE_B, "two waves' rows per tile slot");
   static_assert(GPW * NW == BN / 4, "tile groups must split over the waves");
   __shared__ __attribute__((aligned(1024))) char smem[4 * TILE_B];  // K slot 0, K slot 1, V slot 0, V slot 1
 
@@ -71,13 +73,7 @@ attn_fwd_d256_pipe_kernel(AttnParams p) {
   const char* vp = reinterpret_cast<const char*>(static_cast<const S*>(p.v) + b * p.v_sb + hk * p.v_sh);
   const int64_t k_ss_b = p.k_ss * (int64_t)sizeof(S), v_ss_b = p.v_ss * (int64_t)sizeof(S);
 
-  // Q fragments, all loads back to back (a row past the end reads the last row and is zeroed below).
   V8 qf[D / 16];
-  {
-    const int qr = min(qi, p.Sq - 1);
-#pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) qf[kk] = ld16<V8>(qp + (int64_t)qr * p.q_ss + 16 * kk + 8 * g);
-  }
 
   // Key tiles of the workgroup and of this wave.
   const int q_last = min(q0 + BM, p.Sq) - 1;
@@ -429,9 +425,25 @@ attn_fwd_d256_pipe_kernel(AttnParams p) {
 #pragma unroll
   for (int mb = 0; mb < NMB; ++mb) scur[mb] = snext[mb] = f32x16{};
   if (t_begin < t_end) {
+    // Q through the LDS, in the tiles' layout, a wave's 32 rows (half a tile) in slot 1 of the K ring (waves 0, 1) or of
+    // the V ring (2, 3), which no first copy fills; K(t_begin + 1) follows once every wave has read its rows. Fragments
+    // loaded straight from global memory take 16 loads per wave with 64 lanes on 32 rows each, ~64 cycles of address
+    // processing per load. Rows past the end read the last row.
+    const uint32_t q_slot = smem_base + (uint32_t)((1 + 2 * (w >> 1)) * TILE_B + (w & 1) * QSLOT_B);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int i = 0; i < IPG; ++i) {
+        const int64_t row = min(qw0 + 4 * j + i * RPI + lane / LPR, p.Sq - 1);
+        dma16(q_slot + j * GROUP_B + i * RPI * ROW_B,
+              reinterpret_cast<const char*>(qp + row * p.q_ss) + src_chunk[i] * 16);
+      }
     issue_k(t_begin, 0);
-    if (t_begin + 1 < t_end) issue_k(t_begin + 1, 1);
     issue_v(t_begin, 0);
+    wait_vmem<2 * DMA_PER_TILE>();  // Q has landed
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk)
+      qf[kk] = lds_read<V8>(q_slot + k_lane + 64u * (uint32_t)(((kk >> 1) & 3) ^ s4) + 256 * (kk >> 3) + 32 * (kk & 1));
     // Q: zero the rows past the end, pin the fragments in AGPRs (MFMA reads its B operand from there; the VGPRs
     // stay free for O, the two score tiles and the fragments read ahead).
     const bool live = qi < p.Sq;
@@ -442,9 +454,9 @@ attn_fwd_d256_pipe_kernel(AttnParams p) {
       if constexpr (SOFTCAP) qf[kk] = from_f32x8<V8>(to_f32x8(qf[kk]) * p.sc_a);
       asm volatile("" : "+a"(qf[kk]));
     }
-    if (t_begin + 1 < t_end) wait_vmem<2 * DMA_PER_TILE>();  // K(t_begin) has landed
-    else wait_vmem<DMA_PER_TILE>();
+    wait_vmem<DMA_PER_TILE>();  // K(t_begin) has landed
     __syncthreads();
+    if (t_begin + 1 < t_end) issue_k(t_begin + 1, 1);
     if (t_begin >= wt_begin && t_begin < wt_end) {
       qk(0u, scur);
       if (t_begin >= t_full0 && t_begin < t_full1) prep(t_begin, scur, std::false_type{});
@@ -478,22 +490,29 @@ attn_fwd_d256_pipe_kernel(AttnParams p) {
 
   const float l_tot = half_swap_sum(l_part[0] + l_part[1]);
   const float inv = p.Sk == 0 ? 0.f : 1.0f / l_tot;  // no keys at all: o = 0 (an empty P.V), lse = -inf
-  if (qi < p.Sq) {
-    S* op = static_cast<S*>(p.o) + b * p.o_sb + (int64_t)qi * p.o_ss + h * p.o_sh;
+  // O leaves as whole rows through the LDS (the accumulators hold 4 consecutive elements of a row per lane).
+  __syncthreads();  // every wave is done with the tiles
+  char* o_slot = smem + w * QSLOT_B;
 #pragma unroll
-    for (int db = 0; db < D / 32; ++db) {
+  for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        V4 ov;
+    for (int jj = 0; jj < 4; ++jj) {
+      V4 ov;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ov[e] = to_s<S>(oacc[db][4 * jj + e] * inv);
-        *reinterpret_cast<V4*>(op + db * 32 + 8 * jj + 4 * g) = ov;
-      }
+      for (int e = 0; e < 4; ++e) ov[e] = to_s<S>(oacc[db][4 * jj + e] * inv);
+      *reinterpret_cast<V4*>(o_slot + (r >> 2) * GROUP_B + s4 * ROW_B + 16 * ((4 * db + jj) ^ (4 * s4)) + 8 * g) = ov;
     }
-    if (p.lse != nullptr && g == 0) {
-      const float lse2 = m_run == -INFINITY ? -INFINITY : m_run * c + fast_log2(l_tot);
-      p.lse[(int64_t)bh * p.Sq + qi] = p.lse_base2 ? lse2 : lse2 * kLn2;
-    }
+  if (p.lse != nullptr && g == 0 && qi < p.Sq) {
+    const float lse2 = m_run == -INFINITY ? -INFINITY : m_run * c + fast_log2(l_tot);
+    p.lse[(int64_t)bh * p.Sq + qi] = p.lse_base2 ? lse2 : lse2 * kLn2;
+  }
+  S* ob = static_cast<S*>(p.o) + b * p.o_sb + h * p.o_sh;
+#pragma unroll
+  for (int i = 0; i < 32 / RPI; ++i) {
+    const int row = i * RPI + lane / LPR, chunk = lane % LPR;
+    const V8 ov = *reinterpret_cast<const V8*>(o_slot + (row >> 2) * GROUP_B + (row & 3) * ROW_B +
+                                               16 * (chunk ^ (4 * (row & 3))));
+    if (qw0 + row < p.Sq) *reinterpret_cast<V8*>(ob + (int64_t)(qw0 + row) * p.o_ss + 8 * chunk) = ov;
   }
 }
 

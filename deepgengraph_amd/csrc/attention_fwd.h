@@ -71,7 +71,7 @@ attn_fwd_dma_kernel(AttnParams p) {
   // constant column e_0 and whose B fragment holds -m in k-slot 0. The accumulator then holds s*c - m and
   // P = exp2(acc) needs no per-element arithmetic. The reference maxima are bf16 values so that -m is exact in
   // the B operand; the pre-scaled Q carries the same 2^-9 relative rounding as the reference's bf16 scores.
-  constexpr bool BIAS = D >= 128 && FASTSUM && !SOFTCAP && !REFROUND && std::is_same<T, BF16>::value;
+  constexpr bool BIAS = D == 128 && FASTSUM && !SOFTCAP && !REFROUND && std::is_same<T, BF16>::value;
   V8 abias = V8{};
   abias[0] = g == 0 ? to_s<S>(1.0f) : to_s<S>(0.0f);
   V8 bbias[NQB];
@@ -645,11 +645,14 @@ void launch_fwd_d128(const AttnParams& p, hipStream_t st) {
   launch_fwd_form<T, 128, 8, 1, 128, 2, 2, MASK, SOFTCAP, REFROUND>(p, st);
 }
 
-// head_dim 256: 4 waves x 32 rows (one wave per SIMD). Scores kept in fp32 run on the software-pipelined kernel of
-// attention_d256.hip, reference-rounded ones on the direct-load kernel with 64-key tiles in a 2-stage ring.
+// head_dim 256: 4 waves of one per SIMD. Scores kept in fp32 run on the software-pipelined kernel of attention_d256.hip
+// (128 rows per workgroup), except where 64-row workgroups, two waves to the same rows (KG 2), are at most one per CU:
+// these halve the serial chain of a row (bf16, soft-cap, 16 / 8 heads: S=256 15.0 -> 12.3 us, S=512 21.4 -> 17.5,
+// S=1024 36.0 -> 28.4; 2 x 1280, 640 of them, stays at 47). Reference-rounded scores run on the direct-load kernel.
 template <typename T, bool MASK, bool SOFTCAP, int REFROUND>
 void launch_fwd_d256(AttnParams p, hipStream_t st) {
   if constexpr (REFROUND == 0) {
+    if (fwd_groups(p, 64) <= kCUs) return launch_fwd_form<T, 256, 4, 2, 64, 2, 1, MASK, SOFTCAP, REFROUND>(p, st);
     p.n_tiles = (p.Sq + 127) / 128;
     launch_attn_d256_pipe(p, std::is_same<T, BF16>::value, st);
   } else {

@@ -95,10 +95,11 @@ def test_prefill_d256_gqa_large_kv_order(gpu, B, Sq, Sk, Hq, Hkv, dtype, causal,
         assert_close(out[:, :, h:h + 1].float(), ref.float(), *TOL[dtype], what)
 
 
-# Every form of the head_dim 64 / 128 forward (rows per workgroup and waves per row block, chosen by the number of
+# Every form of the 16-bit forward (rows per workgroup and waves per row block, chosen by the number of
 # workgroups a launch has): heads, the few that are checked are whole. Sizes at the edges of 32-row blocks and 32 / 128-key
 # tiles, rows that see no key (Sq > Sk), tiles whose key groups are partly or wholly past the end, masks on both sides.
-FORM_HEADS = [(64, 4), (64, 60), (64, 200), (128, 8), (128, 96), (128, 288)]
+FORM_HEADS = [(64, 4), (64, 60), (64, 200), (128, 8), (128, 96), (128, 288),
+              (256, 8), (256, 80)]
 FORM_SHAPES = [
     # Sq, Sk, causal, softcap, window, dtype
     (200, 333, True, 0.0, 0, torch.bfloat16),
