@@ -451,6 +451,9 @@ def nonzero(x: torch.Tensor) -> torch.Tensor:
     return coords[: int(total.item())]
 
 
+TOPK_TWO_STAGE_N = 14336
+
+
 def topk_indices(scores: torch.Tensor, k: int, largest: bool = True) -> torch.Tensor:
     """deepgengraph_exp/cases/models/h2o.py:51-52 (torch.topk then sort of the indices) with a defined tie
     order: the k largest (largest=False: smallest, models/roco.py:55) of each row of scores [..., n] (fp32), ties
@@ -462,7 +465,9 @@ def topk_indices(scores: torch.Tensor, k: int, largest: bool = True) -> torch.Te
     n = scores.shape[-1]
     rows = scores.numel() // n if n else 0
     out = torch.empty(*scores.shape[:-1], k, dtype=torch.int64, device=scores.device)
-    ws = _select_workspace(rows, n, scores.device)
+    # Rows of up to 65536 keys need no scratch memory; from TOPK_TWO_STAGE_N keys the library splits a row over several
+    # workgroups if it gets some (as much as a row just beyond 65536 keys needs).
+    ws = _select_workspace(rows, max(n, 65537) if n >= TOPK_TWO_STAGE_N and rows <= 256 else n, scores.device)
     _lib.call("dgg_topk_select_ws", _lib.ptr(scores), rows, n, int(k), 1 if largest else 0, _lib.ptr(out),
               _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.stream_handle(dev))
     return out

@@ -137,11 +137,42 @@ __device__ void radix_kstar(const uint32_t (&key)[PER], uint64_t cand, uint32_t 
   remaining_out = remaining;
 }
 
+// Candidates that may be among the k largest. Each wave finds T_w = the ceil(k / 16)-th largest of its lanes' own maxima
+// (24 leading bits, one ballot per bit): at least that many of its candidates are >= T_w, so at least k of the block's
+// are >= T = min T_w, and those below T drop out. The radix passes that follow are bound by the LDS atomics of a wave's 64
+// lanes on a few hot bins; after this a few lanes per instruction are left. One barrier pair, against ~5 for a pass.
+// For k up to half a lane maximum per thread (beyond, little drops out) and at least 8 keys per lane (top-256 of 32 rows:
+// 1,048,576 keys 142.5 -> 121.6 us, 131,072 25.7 -> 24.4; at 4 keys per lane it costs more than it saves, 2,048 keys
+// 7.3 -> 8.1). Every thread calls this with the same k.
+template <int PER>
+__device__ uint64_t radix_prefilter(const uint32_t (&key)[PER], uint64_t cand, uint32_t k, TopkShared& sh) {
+  if (PER < 8 || k > kTopkThreads / 2) return cand;
+  const uint32_t r = (k + kTopkWaves - 1) / kTopkWaves;
+  uint32_t mx = 0, t = 0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) mx = max(mx, (cand >> j) & 1 ? key[j] : 0u);
+#pragma unroll
+  for (int b = 31; b >= 8; --b) {
+    const uint32_t trial = t | (1u << b);
+    if ((uint32_t)__popcll(__ballot(mx >= trial)) >= r) t = trial;
+  }
+  if ((threadIdx.x & 63) == 0) sh.wsum[threadIdx.x >> 6] = t;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kTopkWaves; ++w) t = min(t, sh.wsum[w]);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+    if (key[j] < t) cand &= ~(1ull << j);
+  return cand;
+}
+
 template <int PER>
 __device__ uint64_t radix_take(const uint32_t (&key)[PER], uint64_t cand, uint32_t k, TopkShared& sh,
                                uint32_t* bound = nullptr) {
   if (k == 0) return 0;
   uint32_t prefix, remaining;
+  cand = radix_prefilter<PER>(key, cand, k, sh);
   radix_kstar<PER>(key, cand, k, sh, prefix, remaining, bound != nullptr);
   if (bound != nullptr && threadIdx.x == 0) {  // K* and how many keys equal to it are taken
     bound[0] = prefix;
@@ -323,6 +354,9 @@ constexpr int kSelNSel = 3;                                 // selections a work
 // with the 64-per-lane merge; 32 keys per lane spill 124 VGPRs and 164 SGPRs).
 constexpr int kSel2Per = 8;                                 // keys per lane in the first stage
 constexpr int kSel2Chunk = 64 * kSel2Per * kTopkWaves;      // keys per workgroup
+// Shortest row that takes the two-stage form by choice. Top-256 of 32 rows, one workgroup per row / two stages, us: 12,288
+// keys 17.2 / 17.7, 16,384 23.0 / 17.0, 32,768 50.8 / 18.1, 65,536 81.9 / 19.0.
+constexpr int kSel2MinN = 14336;
 constexpr int kSel2MaxCand = 64 * kTopkThreads;             // candidates per row
 constexpr int kSel2C2 = 16384;  // second-level candidates per row (groups * k <= 65,536 / 8 + k, see sel2_run)
 
@@ -820,6 +854,7 @@ sel2_local_kernel(KeyF kf, int n, int k, SelWs ws, int cand_sel) {
   }
   if (kk == 0) return;  // (uniform over the workgroup)
   uint32_t kstar, rem;
+  valid = radix_prefilter<kSel2Per>(key, valid, kk, sh);
   radix_kstar<kSel2Per>(key, valid, kk, sh, kstar, rem, false);
   // ranks of the keys equal to K* in index order (wave, step, lane), then the taken keys' slots in the same order
   const uint64_t lt = (1ull << lane) - 1;
@@ -1093,7 +1128,19 @@ extern "C" int64_t dgg_select_workspace_bytes(int64_t rows, int64_t n) {
 
 extern "C" int dgg_topk_select_ws(const float* scores, int64_t rows, int64_t n, int64_t k, int largest,
                                   int64_t* out_idx, void* workspace, int64_t workspace_bytes, void* stream) {
-  if (n <= 65536) return dgg_topk_select(scores, rows, n, k, largest, out_idx, stream);
+  if (n <= 65536) {
+    // Where the caller has scratch memory and the rows alone do not fill the chip, the two-stage form spreads a row over
+    // a workgroup per 8,192 keys (kSel2MinN). Without scratch memory, or with many rows or a large k: one per row.
+    const bool two = n >= kSel2MinN && k >= 1 && k <= 2048 && rows >= 1 && rows <= 256 && scores && out_idx &&
+                     workspace != nullptr && ((uintptr_t)workspace & 255u) == 0 &&
+                     workspace_bytes >= sel_layout(rows, n, nullptr, nullptr);
+    if (!two) return dgg_topk_select(scores, rows, n, k, largest, out_idx, stream);
+    SelWs ws;
+    sel_layout(rows, n, workspace, &ws);
+    sel2_run(KeyScores{scores, (int)n, largest ? 1 : 0}, (int)rows, (int)n, (int)k, ws, kSelAll, out_idx, k,
+             dgg::as_stream(stream));
+    return dgg::check_launch("topk_indices");
+  }
   DGG_REQUIRE(n <= kSelMaxN, DGG_ERR_SHAPE, "topk_indices: n must be <= 2^26 (got %lld)", (long long)n);
   DGG_REQUIRE(rows >= 0, DGG_ERR_SHAPE, "topk_indices: bad row count %lld", (long long)rows);
   DGG_REQUIRE(k >= 1 && k <= n, DGG_ERR_SHAPE, "topk_indices: k must be in [1, n] (got k=%lld, n=%lld)",

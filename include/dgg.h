@@ -242,7 +242,8 @@ int dgg_roco_select(const float* score, const float* sq_score, int64_t rows, int
  * merge, reading the row once; others in radix passes; RoCo's `other` from the boundary of a two-stage `recent`,
  * in two reads of the row) through a caller-provided workspace of
  * dgg_select_workspace_bytes(rows, n) bytes (0 for n <= 65536, where these calls are dgg_topk_select /
- * dgg_roco_select and ignore the workspace), 256-byte aligned; rows <= 65535 when n > 65536. No counterpart in the
+ * dgg_roco_select and need none; a top-k given dgg_select_workspace_bytes(rows, 65537) bytes all the same runs in two
+ * stages where that is faster), 256-byte aligned; rows <= 65535 when n > 65536. No counterpart in the
  * reference beyond the torch.topk calls they replace (models/h2o.py:51, models/snapkv.py:51, models/kf.py:54,
  * models/roco.py:54-61), which have no size limit. */
 int64_t dgg_select_workspace_bytes(int64_t rows, int64_t n);

@@ -336,3 +336,24 @@ def test_column_forms_agree(gpu, S, dtype):
         big = A.keyformer_attention(q, k, v, er, ref_rounding=ref_rounding)[1]
         few = A.keyformer_attention(*some, er[:, hs].contiguous(), ref_rounding=ref_rounding)[1]
         assert_close(big[:, hs].cpu(), few.cpu(), 1e-7, 7e-5, f"keyformer S{S} {dtype} ref={ref_rounding}")
+
+
+@pytest.mark.parametrize("largest", [True, False])
+@pytest.mark.parametrize("n", [14335, 14336, 16385, 40000, 65536])
+def test_topk_two_stages_by_choice(gpu, n, largest):
+    """Rows around and above the length from which topk_indices splits a row over several workgroups, against the
+    one-workgroup form: exact, with ties across the chunks, NaN and infinities, k at the limits of the prefilter."""
+    g = torch.Generator(device=gpu).manual_seed(n)
+    x = torch.randint(0, 3000, (5, n), generator=g, device=gpu).float()
+    x[1] = torch.randn(n, generator=g, device=gpu)
+    x[2] = 1.0
+    x[3, ::7] = float("nan")
+    x[3, 5::11] = float("inf")
+    x[3, 6::11] = -float("inf")
+    x[4] = torch.arange(n, device=gpu).float()
+    lib = _lib.load()
+    for k in (1, 512, 513, 2048):
+        want = torch.empty(5, k, dtype=torch.int64, device=gpu)
+        assert lib.dgg_topk_select(_lib.ptr(x), 5, n, k, int(largest), _lib.ptr(want), _lib.stream_handle(gpu)) == 0
+        got = A.topk_indices(x, k, largest=largest)
+        assert torch.equal(got, want), f"n {n} k {k} largest {largest}"
