@@ -64,14 +64,31 @@ def _splitkv_shaped(Sq: int, Sk: int, Hq: int, Hkv: int, ref_rounding: bool, dty
             and not ref_rounding and dtype in (torch.float16, torch.bfloat16))
 
 
+# Longer query blocks go there too (head_dim 128) while the prefill kernel has at most one 64-row workgroup per CU, so
+# that its time is the serial chain of the keys: up to SPLITKV_WIDE_QLEN query rows, over at least 32 keys per query row
+# (40 beyond 128 rows). Measured on MI355X, bf16, B=1, prefill / split-KV, us: 64 rows 32 / 8 heads 2,048 keys 22.0 / 19.4,
+# 8,192 68 / 36, 32,768 255 / 72; 128 rows 32 heads 4,096 keys 42.7 / 37.6, 32,768 441 / 149, but 2,048 keys 24.1 / 28.8;
+# 256 rows 32 / 8 heads 32,768 keys 260 / 218, but 8,192 keys 71 / 75; 384 rows: never.
+SPLITKV_WIDE_QLEN = 256
+
+
+def _splitkv_wide(B: int, Sq: int, Sk: int, Hq: int, D: int, window, ref_rounding: bool, dtype) -> bool:
+    span = min(Sk, window + Sq - 1) if window else Sk
+    return (D == 128 and 1 <= Sq <= SPLITKV_WIDE_QLEN and span >= max((32 if Sq <= 128 else 40) * Sq, SPLITKV_MIN_KEYS)
+            and B * Hq * (-(-Sq // 64)) <= 256 and not ref_rounding and dtype in (torch.float16, torch.bfloat16))
+
+
 def splitkv_splits(B: int, Sq: int, Hq: int, Hkv: int, span: int) -> int:
     """Key slices for a split-KV call over `span` keys: up to 512 workgroups (1024 for at most 8 rows per KV head, whose
-    partials are small), each slice at least 32 keys and 8 per row it serves, and at most 64 slices below 16K keys, whose
+    partials are small, and for more than 64, whose slices are long), each slice at least 32 keys and 8 per row it serves, and at most 64 slices below 16K keys, whose
     merge would take longer than the keys. The library's own rule for grouped-query decode (splitkv_useful_splits in
     csrc/splitkv.hip, with the measurements)."""
     rows = (Hq // Hkv) * Sq
     groups = max(1, B * Hkv * (-(-rows // (32 if rows <= 32 else 64))))
-    want = -(-(1024 if rows <= 8 else 512) // groups)
+    if rows > 64:  # several row groups read a slice: a multiple of 8 slices keeps them on one XCD and its L2
+        want = max(8, 1024 // groups // 8 * 8)
+    else:
+        want = -(-(1024 if rows <= 8 else 512) // groups)
     min_keys = max(32, 8 * min(rows, 32))
     return int(max(1, min(want, 64 if span < 16384 else 1024, -(-span // min_keys))))
 
@@ -204,7 +221,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool
         if return_lse:
             lse.copy_(lse1.view(B, Hq, 1) * (math.log2(math.e) if lse_base2 else 1.0))
         return (out, lse) if return_lse else out
-    if _splitkv_shaped(Sq, Sk, Hq, Hkv, ref_rounding, q.dtype):
+    if (_splitkv_shaped(Sq, Sk, Hq, Hkv, ref_rounding, q.dtype)
+            or _splitkv_wide(B, Sq, Sk, Hq, D, window, ref_rounding, q.dtype)):
         _splitkv(q, k, v, out, lse, causal, softcap, window, scale, lse_base2, None, dev)
         return (out, lse) if return_lse else out
     flags = ((_lib.ATTN_CAUSAL if causal else 0) | (_lib.ATTN_REF_ROUNDING if ref_rounding else 0)
@@ -467,7 +485,7 @@ def topk_indices(scores: torch.Tensor, k: int, largest: bool = True) -> torch.Te
     out = torch.empty(*scores.shape[:-1], k, dtype=torch.int64, device=scores.device)
     # Rows of up to 65536 keys need no scratch memory; from TOPK_TWO_STAGE_N keys the library splits a row over several
     # workgroups if it gets some (as much as a row just beyond 65536 keys needs).
-    ws = _select_workspace(rows, max(n, 65537) if n >= TOPK_TWO_STAGE_N and rows <= 256 else n, scores.device)
+    ws = _select_workspace(rows, max(n, 65537) if n >= TOPK_TWO_STAGE_N and rows <= 64 else n, scores.device)
     _lib.call("dgg_topk_select_ws", _lib.ptr(scores), rows, n, int(k), 1 if largest else 0, _lib.ptr(out),
               _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.stream_handle(dev))
     return out

@@ -330,11 +330,16 @@ namespace dgg {
 // B=1, 1 row, 32 / 8 heads: 4,001 keys 64: 9.7 (32: 10.8, 8: 22.2); 1,024 keys 32: 7.8 (16: 9.0); 32,768 keys 128: 27.2
 // (64: 29.5, 256: 28.6). B=8, 4,001 keys 16: 28.2 (8: 29.4, 32: 29.7). 16 rows, 32 heads: 8,192 keys 16: 30.8 (8: 39.8,
 // 32: 31.3); 2,048 keys 16: 14.3 (8: 15.9, 32: 16.4). 16 rows, 32 / 8 heads: 8,192 keys 32: 19.1 (16: 23.2, 64: 21.9).
-// 64 rows, 32 heads: 2,048 keys 8: 19.6 (4: 23.7, 16: 22.0).
+// 64 rows, 32 heads: 2,048 keys 8: 19.6 (4: 23.7, 16: 22.0). 128 rows, 32 heads: 32,768 keys 16: 150 (8: 177, 32: 181);
+// 256 rows, 32 / 8 heads: 32,768 keys 32: 72 (16: 93, 64: 91).
 int64_t splitkv_useful_splits(int64_t B, int64_t Sq, int64_t Hq, int64_t Hkv, int64_t span) {
   const int64_t rows = std::max<int64_t>(1, Hq / Hkv * Sq), rpw = rows <= 32 ? 32 : 64;
   const int64_t groups = std::max<int64_t>(1, B * Hkv * ((rows + rpw - 1) / rpw));
-  const int64_t want = ((rows <= 8 ? 1024 : 512) + groups - 1) / groups;
+  // More than 64 rows: several row groups read each slice. Workgroups go round the 8 XCDs by slice first, so a multiple of
+  // 8 slices puts the groups of a slice on one XCD, whose L2 the second finds it in (192 rows, 32 heads, 32,768 keys: 8
+  // slices 207-222 us, 10 285, 11 321; 384 rows, 32 / 8 heads: 16 slices 104, 21 155).
+  const int64_t want = rows > 64 ? std::max<int64_t>(8, 1024 / groups / 8 * 8)
+                                 : ((rows <= 8 ? 1024 : 512) + groups - 1) / groups;
   const int64_t min_keys = std::max<int64_t>(32, 8 * std::min<int64_t>(rows, 32));
   const int64_t cap = span < 16384 ? 64 : 1024;
   return std::max<int64_t>(1, std::min({want, cap, (span + min_keys - 1) / min_keys}));

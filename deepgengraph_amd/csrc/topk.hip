@@ -1131,7 +1131,7 @@ extern "C" int dgg_topk_select_ws(const float* scores, int64_t rows, int64_t n, 
   if (n <= 65536) {
     // Where the caller has scratch memory and the rows alone do not fill the chip, the two-stage form spreads a row over
     // a workgroup per 8,192 keys (kSel2MinN). Without scratch memory, or with many rows or a large k: one per row.
-    const bool two = n >= kSel2MinN && k >= 1 && k <= 2048 && rows >= 1 && rows <= 256 && scores && out_idx &&
+    const bool two = n >= kSel2MinN && k >= 1 && k <= 2048 && rows >= 1 && rows <= 64 && scores && out_idx &&
                      workspace != nullptr && ((uintptr_t)workspace & 255u) == 0 &&
                      workspace_bytes >= sel_layout(rows, n, nullptr, nullptr);
     if (!two) return dgg_topk_select(scores, rows, n, k, largest, out_idx, stream);

@@ -118,3 +118,24 @@ def test_splitkv_rejects_reference_rounding_and_small_workspace(gpu):
     _lib.call("dgg_attn_splitkv", *args(need, _lib.ATTN_CAUSAL))
     torch.cuda.synchronize()
     assert_close(o.cpu().float(), oa.attention(q.cpu(), k.cpu(), v.cpu(), causal=True).float(), 1e-2, 5e-3, "raw ABI")
+
+
+@pytest.mark.parametrize("Sq,Sk,Hq,Hkv,window,routed", [
+    (64, 2100, 16, 4, 0, True),        # 256 rows per KV head
+    (128, 4099, 4, 4, 0, True),        # two 64-row groups, ragged last slice
+    (129, 5160, 4, 2, 0, True),        # 40 keys per row
+    (129, 5159, 4, 2, 0, False),       # one key less
+    (100, 6000, 4, 2, 3200, True),     # a window of 32 keys per row
+    (100, 6000, 4, 2, 900, False),     # a shorter one
+])
+def test_wide_query_blocks(gpu, Sq, Sk, Hq, Hkv, window, routed):
+    """Query blocks of 64 to 256 rows around the line from which attention() takes the split-KV kernels: the same result
+    on either side of it, with soft-cap and lse."""
+    assert A._splitkv_wide(1, Sq, Sk, Hq, 128, window, False, torch.bfloat16) == routed
+    g = torch.Generator().manual_seed(Sq + Sk)
+    q = torch.randn(1, Sq, Hq, 128, generator=g).bfloat16()
+    k, v = (torch.randn(1, Sk, Hkv, 128, generator=g).bfloat16() for _ in range(2))
+    out, lse = A.attention(q.to(gpu), k.to(gpu), v.to(gpu), window=window, softcap=30.0, return_lse=True)
+    ref, ref_lse = oa.attention(q, k, v, causal=True, window=window or None, softcap=30.0, return_lse=True)
+    assert_close(out.cpu().float(), ref.float(), 2e-2, 1e-2, "out")
+    assert_close(lse.cpu(), ref_lse, 2e-2, 1e-2, "lse")
