@@ -137,10 +137,12 @@ def ptr(t: torch.Tensor | None):
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def stream_handle(device: torch.device):
-    """The current stream of the device, as the address the library takes (0 / None: the null stream)."""
-    if _raw_stream is not None and device.index is not None:
-        return _raw_stream(device.index)
+def stream_handle(device):
+    """The current stream of a device (a torch.device, an index, or whatever torch.cuda.current_stream takes), as the
+    address the library takes (0: the null stream)."""
+    index = getattr(device, "index", device)
+    if _raw_stream is not None and type(index) is int:
+        return _raw_stream(index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
