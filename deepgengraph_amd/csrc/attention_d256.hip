@@ -444,19 +444,22 @@ attn_fwd_d256_pipe_kernel(AttnParams p) {
 #pragma unroll
     for (int kk = 0; kk < D / 16; ++kk)
       qf[kk] = lds_read<V8>(q_slot + k_lane + 64u * (uint32_t)(((kk >> 1) & 3) ^ s4) + 256 * (kk >> 3) + 32 * (kk & 1));
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(qf[kk]));
+    __syncthreads();  // every wave has its rows: slot 1 of the K ring is free
+    if (t_begin + 1 < t_end) issue_k(t_begin + 1, 1);
     // Q: zero the rows past the end, pin the fragments in AGPRs (MFMA reads its B operand from there; the VGPRs
     // stay free for O, the two score tiles and the fragments read ahead).
     const bool live = qi < p.Sq;
 #pragma unroll
     for (int kk = 0; kk < D / 16; ++kk) {
-      asm volatile("" : "+v"(qf[kk]));
       if (!live) qf[kk] = V8{};
       if constexpr (SOFTCAP) qf[kk] = from_f32x8<V8>(to_f32x8(qf[kk]) * p.sc_a);
       asm volatile("" : "+a"(qf[kk]));
     }
-    wait_vmem<DMA_PER_TILE>();  // K(t_begin) has landed
+    if (t_begin + 1 < t_end) wait_vmem<2 * DMA_PER_TILE>();  // K(t_begin) has landed
+    else wait_vmem<DMA_PER_TILE>();
     __syncthreads();
-    if (t_begin + 1 < t_end) issue_k(t_begin + 1, 1);
     if (t_begin >= wt_begin && t_begin < wt_end) {
       qk(0u, scur);
       if (t_begin >= t_full0 && t_begin < t_full1) prep(t_begin, scur, std::false_type{});
