@@ -23,8 +23,8 @@ using namespace dgg_attn;
 // Forward kernel: NW waves of 32 query rows over a ring of NSTAGE tiles of BN keys. KG: waves that share the same 32
 // rows, each taking BN / KG keys of every tile (its own running maximum, row sum and O, combined through the LDS at the
 // end), so a workgroup covers 32 * NW / KG rows. OCC: waves per SIMD the register budget is sized for. FASTSUM: the row
-// sums add the 16-bit rounded probabilities two at a time (v_dot2); used when no lse is written, since the O
-// normalisation tolerates the rounding but the column-sum pass needs the fp32 row sums.
+// sums add the 16-bit rounded probabilities two at a time (v_dot2); used at head_dim 128 and 256 when no lse is written,
+// since the O normalisation tolerates the rounding but the column-sum pass needs the fp32 row sums.
 template <typename T, int D, int NW, int KG, int BN, int NSTAGE, int OCC, bool MASK, bool SOFTCAP, int REFROUND, bool FASTSUM>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 attn_fwd_dma_kernel(AttnParams p) {
@@ -597,12 +597,15 @@ void launch_fwd_form(AttnParams p, hipStream_t st) {
   constexpr int BM = 32 * NW / KG;
   p.n_tiles = (p.Sq + BM - 1) / BM;
   const unsigned grid = (unsigned)p.n_tiles * p.B * p.Hq;
-  if (!REFROUND && p.lse == nullptr)
-    hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, KG, BN, NS, OCC, MASK, SOFTCAP, REFROUND, !REFROUND>), dim3(grid),
-                       dim3(64 * NW), 0, st, p);
-  else
-    hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, KG, BN, NS, OCC, MASK, SOFTCAP, REFROUND, false>), dim3(grid),
-                       dim3(64 * NW), 0, st, p);
+  if constexpr (!REFROUND && D != 64) {
+    if (p.lse == nullptr) {
+      hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, KG, BN, NS, OCC, MASK, SOFTCAP, REFROUND, true>), dim3(grid),
+                         dim3(64 * NW), 0, st, p);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, KG, BN, NS, OCC, MASK, SOFTCAP, REFROUND, false>), dim3(grid),
+                     dim3(64 * NW), 0, st, p);
 }
 
 // Workgroups of a launch with bm query rows each.
@@ -612,7 +615,8 @@ constexpr int kCUs = 256;
 // head_dim 64. Large launches: 4 waves x 32 rows, 64-key tiles, 2 stages (32 KiB: three workgroups per CU at three
 // waves per SIMD). The loop is bound by vector issue (a 32 x 32 block of scores takes 8 MFMAs and ~26 x 16 lanes of
 // exp / fma / max / pack), and more waves hide more of it: fp16, B=8, S=1000, H=16 without a mask 60.4 -> 47.7 us
-// against the kernel that staged tiles through registers; two workgroups of 8 waves 56 us, 64 rows per wave 49 us.
+// against the kernel that staged tiles through registers; two workgroups of 8 waves 56 us, 64 rows per wave 49 us. The
+// row sums are always of the fp32 probabilities (FASTSUM would gain nothing: 47.2 us either way).
 // Launches that leave the chip idle split each tile's keys over KG waves instead: 32-row workgroups of 4 waves (KG 4)
 // while one per CU suffices (1 x 300 x 16: 8.3 -> 6.4 us), 64-row workgroups of 8 waves (KG 4) up to one per CU
 // (1 x 1024 x 16: 16.4 -> 11.3 us), and also up to two per CU when the rows are long (1 x 2048 x 16: 29.6 -> 27.2 us,

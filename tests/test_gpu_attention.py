@@ -131,6 +131,18 @@ def test_prefill_forms(gpu, D, H, Sq, Sk, causal, softcap, window, dtype, with_l
         assert_close(lse_c[fin], ref_lse[fin], 2e-2, 1e-2, what + " lse")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H", [4, 60, 200])
+def test_prefill_d64_row_sums_are_fp32(gpu, H, dtype):
+    """head_dim 64 normalises O by the fp32 sum of the fp32 probabilities whether or not the lse is asked for (that sum is
+    the lse's), in each of its forms: the same output to the bit."""
+    q, k, v = (t.to(gpu) for t in _qkv(1, 200, 333, H, H, 64, dtype, seed=H))
+    for causal, softcap in ((True, 0.0), (False, 0.0), (True, 30.0)):
+        out = A.attention(q, k, v, causal=causal, softcap=softcap)
+        with_lse, _ = A.attention(q, k, v, causal=causal, softcap=softcap, return_lse=True)
+        assert torch.equal(out, with_lse), f"H{H} {dtype} causal={causal} cap={softcap}"
+
+
 def test_prefill_two_rounds_of_unequal_rows(gpu):
     """Causal rows of one 256-row workgroup per CU at most: the 128-row form in two rounds."""
     S, H = 1000, 40
