@@ -271,7 +271,8 @@ attn_kf_rowlse_dma_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(1024))) char smem[2 * KT_B + NW * ET_B];
 
   int qt, bh;
-  map_block<true>(p.n_tiles, p.B * p.Hq, true, qt, bh);
+  const int bid = p.block0 + blockIdx.x;
+  map_block<true>(p.n_tiles, p.B * p.Hq, true, qt, bh, bid);
   const int b = bh / p.Hq, h = bh - b * p.Hq;
   const int hk = h / p.group;
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, g = lane >> 5;
@@ -302,7 +303,7 @@ attn_kf_rowlse_dma_kernel(AttnParams p) {
   if (p.window > 0) k_begin = max(0, q0 + p.offset - p.window + 1);
   const int t_begin = k_begin / BN;
   const int n_t = k_end > k_begin ? (k_end + BN - 1) / BN - t_begin : 0;
-  const int rot = n_t > 0 ? (int)((blockIdx.x >> 3) * 7 % n_t) : 0;
+  const int rot = n_t > 0 ? (int)((unsigned)(bid >> 3) * 7 % n_t) : 0;
   auto tile_of = [&](int i) { return t_begin + (i + rot < n_t ? i + rot : i + rot - n_t); };
   int k_hi = p.Sk - 1, k_lo = 0;
   if (p.causal) k_hi = min(k_hi, qi + p.offset);
@@ -645,7 +646,7 @@ attn_colsum_d128_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(1024))) char smem[NSTAGE * STAGE_B];
 
   int kt, bh;
-  map_block<OCC == 4>(p.n_tiles, p.B * p.Hq, false, kt, bh);
+  map_block<OCC == 4>(p.n_tiles, p.B * p.Hq, false, kt, bh, p.block0 + blockIdx.x);
   const int b = bh / p.Hq, h = bh - b * p.Hq;
   const int hk = h / p.group;
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, g = lane >> 5;
@@ -967,17 +968,21 @@ void launch_colsum(AttnParams p, hipStream_t st) {
   hipLaunchKernelGGL((attn_colsum_kernel<T, D, MASK, SOFTCAP, REFROUND, EPI>), dim3(grid), dim3(kThreads), 0, st, p);
 }
 
+constexpr int kColMinKeys = 64;  // fewest keys per workgroup of a column pass
+
 template <typename T, int NG, int OCC, bool MASK, bool SOFTCAP, int REFROUND, int EPI>
 void launch_colsum_d128_form(AttnParams p, hipStream_t st) {
   constexpr int NW = 8, BQ = 128, BK = 32 * NW / NG;
+  static_assert(BK >= kColMinKeys, "check_blocks");
   p.n_tiles = (p.Sk + BK - 1) / BK;
-  const unsigned grid = (unsigned)p.n_tiles * p.B * p.Hq;
-  if (p.lse_base2)
-    hipLaunchKernelGGL((attn_colsum_d128_kernel<T, NW, NG, BQ, OCC, MASK, SOFTCAP, REFROUND, true, EPI>), dim3(grid),
-                       dim3(64 * NW), 0, st, p);
-  else
-    hipLaunchKernelGGL((attn_colsum_d128_kernel<T, NW, NG, BQ, OCC, MASK, SOFTCAP, REFROUND, false, EPI>), dim3(grid),
-                       dim3(64 * NW), 0, st, p);
+  launch_blocks(p, 64 * NW, [&](unsigned grid, const AttnParams& p) {
+    if (p.lse_base2)
+      hipLaunchKernelGGL((attn_colsum_d128_kernel<T, NW, NG, BQ, OCC, MASK, SOFTCAP, REFROUND, true, EPI>), dim3(grid),
+                         dim3(64 * NW), 0, st, p);
+    else
+      hipLaunchKernelGGL((attn_colsum_d128_kernel<T, NW, NG, BQ, OCC, MASK, SOFTCAP, REFROUND, false, EPI>), dim3(grid),
+                         dim3(64 * NW), 0, st, p);
+  });
 }
 
 // head_dim 128 column passes: 8 waves, 128-row query tiles; 64 keys per workgroup in four row groups (NG 4) or 128 in
@@ -1035,14 +1040,16 @@ void pick_col(const AttnParams& p, bool ref, int epi, hipStream_t st) {
 
 template <typename T, int D, bool MASK, int REFROUND>
 void launch_kf_rowlse(const AttnParams& p, bool vec, hipStream_t st) {
-  const unsigned grid = (unsigned)p.n_tiles * p.B * p.Hq;
   if constexpr (D == 128) {
     // exp_rand as whole 16-byte chunks: aligned rows and a key count that ends on a chunk
     if (vec && p.Sk % 4 == 0) {
-      hipLaunchKernelGGL((attn_kf_rowlse_dma_kernel<T, MASK, REFROUND>), dim3(grid), dim3(512), 0, st, p);
+      launch_blocks(p, 512, [&](unsigned grid, const AttnParams& p) {
+        hipLaunchKernelGGL((attn_kf_rowlse_dma_kernel<T, MASK, REFROUND>), dim3(grid), dim3(512), 0, st, p);
+      });
       return;
     }
   }
+  const unsigned grid = (unsigned)p.n_tiles * p.B * p.Hq;
   if (vec) hipLaunchKernelGGL((attn_kf_rowlse_kernel<T, D, MASK, REFROUND, true>), dim3(grid), dim3(kThreads), 0, st, p);
   else hipLaunchKernelGGL((attn_kf_rowlse_kernel<T, D, MASK, REFROUND, false>), dim3(grid), dim3(kThreads), 0, st, p);
 }
@@ -1160,6 +1167,7 @@ int prefill_impl(const char* op, const void* q, const void* k, const void* v, vo
   hipStream_t st = dgg::as_stream(stream);
   // Sk == 0 still launches and writes o = 0 (the reference's P.V over an empty key axis) and lse = -inf.
   if (dtype == DGG_F32) {  // fp32 has no 16-bit rounding point: reference rounding changes nothing
+    if (int rc = check_blocks(op, Sq, kF32Rows, B, Hq)) return rc;
     launch_attn_f32_fwd(p, (int)D, st);
     return dgg::check_launch(op);
   }
@@ -1227,6 +1235,7 @@ int colscore(const char* op, const void* q, const void* k, const float* lse, int
               epi);
   DGG_REQUIRE(epi == kColSum || softcap == 0.f, DGG_ERR_UNSUPPORTED, "%s: epilogue %d takes no soft-cap", op, epi);
   if (B == 0 || Sk == 0) return DGG_OK;
+  if (int rc = check_blocks(op, Sk, kColMinKeys, B, Hq)) return rc;
   if (epi == kColAnyGe) {
     DGG_REQUIRE(out_any != nullptr, DGG_ERR_NULL, "%s: null output pointer", op);
     DGG_REQUIRE(Sq == 0 || thr != nullptr, DGG_ERR_NULL, "%s: null threshold pointer", op);
@@ -1335,6 +1344,7 @@ extern "C" int dgg_attn_kf_colsum(const void* q, const void* k, const float* exp
               "%s: dtype code %d not supported (the KeyFormer passes take f16 or bf16)", op, dtype);
   if (int rc = validate_attn(op, q, k, B, Sq, Sk, Hq, Hkv, D, strides, 6, scale, 0.f, window, dtype)) return rc;
   if (B == 0 || Sk == 0) return DGG_OK;
+  if (int rc = check_blocks(op, Sk, kColMinKeys, B, Hq)) return rc;
   DGG_REQUIRE(kf_score != nullptr, DGG_ERR_NULL, "%s: null output", op);
   DGG_REQUIRE(Sq == 0 || lse2 != nullptr, DGG_ERR_NULL, "%s: null lse pointer", op);
   if (Sq > 0)

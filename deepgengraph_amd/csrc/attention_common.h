@@ -12,7 +12,8 @@ namespace dgg_attn {
 
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
-constexpr int kBM = 32 * kWaves;  // query rows per forward workgroup
+constexpr int kBM = 32 * kWaves;  // query rows per workgroup of KeyFormer's row pass
+constexpr int kF32Rows = 16;      // query rows per workgroup of the fp32 forward
 constexpr float kRescaleThreshold = 8.0f;  // log2 units
 
 
@@ -51,6 +52,7 @@ struct AttnParams {
   float sc_a;    // 2 * scale / softcap * log2(e)
   float sc_b;    // softcap * log2(e)
   const float* rope_cs;  // fused rotary of the query rows: [B * Sq, D] (cos | sin) per row, or nullptr
+  int block0;            // first workgroup of this launch (launch_blocks)
 };
 
 // Probability of the perturbed score for KeyFormer: x2 = the score in the exp2 domain, e = exp_rand, l2 = the
@@ -161,14 +163,14 @@ __device__ __forceinline__ f16x2 ref_scores_f16(float a, float b, const AttnPara
   return __builtin_convertvector(f32x2{q0, q1}, f16x2);
 }
 
-// Maps blockIdx.x to (tile, batch*head). Longest tiles first; when the (batch, head) count divides by 8,
+// Maps a workgroup's number to (tile, batch*head). Longest tiles first; when the (batch, head) count divides by 8,
 // each XCD gets a contiguous group of heads so their K/V are shared through that XCD's L2.
 // PAIR, for kernels of which a CU holds two workgroups: a launch of between one and two per CU is resident at once, the
 // workgroups after the first 256 joining them in order. Taking those from the short end gives every CU a long and a
 // short tile, not the i-th longest and the (i + 256)-th.
 template <bool PAIR = false>
-__device__ __forceinline__ void map_block(int n_tiles, int bh_count, bool reverse, int& tile, int& bh) {
-  const int bid = blockIdx.x;
+__device__ __forceinline__ void map_block(int n_tiles, int bh_count, bool reverse, int& tile, int& bh,
+                                          int bid = blockIdx.x) {
   const bool pair = PAIR && n_tiles * bh_count > 256 && n_tiles * bh_count <= 512;
   int t_major, bh_minor;
   if ((bh_count & 7) == 0) {
@@ -336,6 +338,23 @@ template <int D, bool SOFTCAP, typename F>
 void with_ref_mode(bool ref, const AttnParams& p, F&& f) {
   if (ref) f(std::integral_constant<int, 1>{});
   else f(std::integral_constant<int, 0>{});
+}
+
+// Launches the n_tiles * B * Hq workgroups of p: launch(grid, p) with p.block0 set, for kernels that take their number as
+// block0 + blockIdx.x. A launch takes fewer than 2^32 work-items, so a larger one goes out in parts (of a multiple of 8
+// workgroups, which leaves each on its XCD). check_blocks: the limit on the count itself, for the entry points.
+template <typename F>
+void launch_blocks(AttnParams p, int threads, F&& launch) {
+  const int64_t total = (int64_t)p.n_tiles * p.B * p.Hq, most = (1ll << 32) / threads - 8;
+  for (int64_t b0 = 0; b0 < total; b0 += most) {
+    p.block0 = (int)b0;
+    launch((unsigned)std::min(most, total - b0), p);
+  }
+}
+inline int check_blocks(const char* op, int64_t rows, int rows_per_block, int64_t B, int64_t Hq) {
+  DGG_REQUIRE((rows + rows_per_block - 1) / rows_per_block * B * Hq < (1ll << 31), DGG_ERR_SHAPE,
+              "%s: grid too large", op);
+  return DGG_OK;
 }
 
 // Host-side validation of the attention arguments shared by the prefill, column and split-KV entry points

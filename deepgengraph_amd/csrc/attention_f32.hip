@@ -70,6 +70,7 @@ constexpr int kKG = 4;
 
 template <int D, bool SOFTCAP>
 __global__ void __launch_bounds__(64 * kKG) attn_fwd_f32_kernel(AttnParams p) {
+  static_assert(kF32Rows == 16, "one row per lane of 16");
   constexpr int NC = D / 16;             // 16-byte chunks of a fragment; 16-wide head-dim blocks of O^T
   constexpr int RS = D + 4;              // LDS row (floats): 16 rows of one chunk on distinct banks
   constexpr int SLOT = 16 * RS, OSLOT = NC * 64 * 4;  // floats: a wave's K block (at the start, Q); its O at the end
@@ -77,7 +78,7 @@ __global__ void __launch_bounds__(64 * kKG) attn_fwd_f32_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(16))) float smem[SMEM];
 
   int qt, bh;
-  map_block(p.n_tiles, p.B * p.Hq, true, qt, bh);
+  map_block(p.n_tiles, p.B * p.Hq, true, qt, bh, p.block0 + blockIdx.x);
   const int b = bh / p.Hq, h = bh - b * p.Hq, hk = h / p.group;
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
   const int kg = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -302,10 +303,11 @@ __global__ void __launch_bounds__(kThr) attn_col_f32_kernel(AttnParams p) {
 
 template <int D>
 void fwd_f32(AttnParams p, hipStream_t st) {
-  p.n_tiles = (p.Sq + 15) / 16;
-  const unsigned grid = (unsigned)p.n_tiles * p.B * p.Hq;
-  if (p.softcap > 0.f) hipLaunchKernelGGL((attn_fwd_f32_kernel<D, true>), dim3(grid), dim3(64 * kKG), 0, st, p);
-  else hipLaunchKernelGGL((attn_fwd_f32_kernel<D, false>), dim3(grid), dim3(64 * kKG), 0, st, p);
+  p.n_tiles = (p.Sq + kF32Rows - 1) / kF32Rows;
+  launch_blocks(p, 64 * kKG, [&](unsigned grid, const AttnParams& p) {
+    if (p.softcap > 0.f) hipLaunchKernelGGL((attn_fwd_f32_kernel<D, true>), dim3(grid), dim3(64 * kKG), 0, st, p);
+    else hipLaunchKernelGGL((attn_fwd_f32_kernel<D, false>), dim3(grid), dim3(64 * kKG), 0, st, p);
+  });
 }
 template <int D, bool SOFTCAP, int EPI>
 void launch_col_f32_d(const AttnParams& p, hipStream_t st) {

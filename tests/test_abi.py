@@ -89,6 +89,21 @@ def test_prefill_validation(lib):
     assert _prefill(lib, Sk=0, k=None, v=None, q=None) == E_NULL
 
 
+def test_grid_limits(lib):
+    # 2^31 workgroups or more are refused by name: 16 query rows each in fp32, 64 keys each in the column passes (128 rows
+    # or keys are what the common check counts)
+    st = _strides([0, 64, 0] * 4)
+    big = dict(B=1 << 10, Hq=1 << 5, Hkv=1, D=64, strides=st)
+    assert _prefill(lib, dtype=_lib.DGG_F32, Sq=1 << 20, Sk=1, **big) == E_SHAPE
+    assert b"grid too large" in lib.dgg_last_error()
+    s = _strides([0, 128, 0] * 2)
+    assert lib.dgg_attn_colsum(FAKE, FAKE, FAKE, FAKE, 1 << 10, 1, 1 << 22, 1 << 5, 1, 128, s, 0.1, 0.0, 0, 0,
+                               _lib.DGG_F16, None) == E_SHAPE
+    er = _strides([0, 0, 1 << 22])
+    assert lib.dgg_attn_kf_colsum(FAKE, FAKE, FAKE, er, FAKE, FAKE, 1 << 10, 1, 1 << 22, 1 << 5, 1, 128, s, 0.1,
+                                  1.5, 0, 0, _lib.DGG_F16, None) == E_SHAPE
+
+
 def test_colsum_validation(lib):
     s = _strides([128 * 512, 512, 128] * 2)
     assert lib.dgg_attn_colsum(FAKE, FAKE, None, FAKE, 1, 64, 64, 2, 2, 128, s, 0.1, 0.0, 0, 1, _lib.DGG_F16,
