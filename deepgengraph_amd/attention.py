@@ -80,9 +80,10 @@ def _splitkv_wide(B: int, Sq: int, Sk: int, Hq: int, D: int, window, ref_roundin
 
 def splitkv_splits(B: int, Sq: int, Hq: int, Hkv: int, span: int) -> int:
     """Key slices for a split-KV call over `span` keys: up to 512 workgroups (1024 for at most 8 rows per KV head, whose
-    partials are small, and for more than 64, whose slices are long), each slice at least 32 keys and 8 per row it serves, and at most 64 slices below 16K keys, whose
-    merge would take longer than the keys. The library's own rule for grouped-query decode (splitkv_useful_splits in
-    csrc/splitkv.hip, with the measurements)."""
+    partials are small, and for more than 64, whose slices are long), each slice at least 32 keys and 8 per row it
+    serves, and at most 64 slices below 16K keys, whose merge would take longer than the keys. Beyond 64 rows per KV head
+    a multiple of 8. The library's own rule for grouped-query decode (splitkv_useful_splits in csrc/splitkv.hip, with the
+    measurements)."""
     rows = (Hq // Hkv) * Sq
     groups = max(1, B * Hkv * (-(-rows // (32 if rows <= 32 else 64))))
     if rows > 64:  # several row groups read a slice: a multiple of 8 slices keeps them on one XCD and its L2
@@ -90,7 +91,10 @@ def splitkv_splits(B: int, Sq: int, Hq: int, Hkv: int, span: int) -> int:
     else:
         want = -(-(1024 if rows <= 8 else 512) // groups)
     min_keys = max(32, 8 * min(rows, 32))
-    return int(max(1, min(want, 64 if span < 16384 else 1024, -(-span // min_keys))))
+    n = int(max(1, min(want, 64 if span < 16384 else 1024, -(-span // min_keys))))
+    if rows <= 64 or n < 8:
+        return n
+    return n // 8 * 8 if groups * (n // 8 * 8) >= 256 else -(-n // 8) * 8
 
 
 def decode_splits(B: int, Hq: int, L: int) -> int:

@@ -337,12 +337,16 @@ int64_t splitkv_useful_splits(int64_t B, int64_t Sq, int64_t Hq, int64_t Hkv, in
   const int64_t groups = std::max<int64_t>(1, B * Hkv * ((rows + rpw - 1) / rpw));
   // More than 64 rows: several row groups read each slice. Workgroups go round the 8 XCDs by slice first, so a multiple of
   // 8 slices puts the groups of a slice on one XCD, whose L2 the second finds it in (192 rows, 32 heads, 32,768 keys: 8
-  // slices 207-222 us, 10 285, 11 321; 384 rows, 32 / 8 heads: 16 slices 104, 21 155).
+  // slices 207-222 us, 10 285, 11 321; 384 rows, 32 / 8 heads: 16 slices 104, 21 155). A span short of whole multiples
+  // rounds down to one, or up where that leaves less than a workgroup per CU (256 rows, 32 / 8 heads: 2,100 keys 9
+  // slices 23.8, 8 20.3; 3,000 keys 12 25.1, 8 22.3; 80 rows: 3,000 keys 12 17.0, 8 18.3, 16 15.9).
   const int64_t want = rows > 64 ? std::max<int64_t>(8, 1024 / groups / 8 * 8)
                                  : ((rows <= 8 ? 1024 : 512) + groups - 1) / groups;
   const int64_t min_keys = std::max<int64_t>(32, 8 * std::min<int64_t>(rows, 32));
   const int64_t cap = span < 16384 ? 64 : 1024;
-  return std::max<int64_t>(1, std::min({want, cap, (span + min_keys - 1) / min_keys}));
+  const int64_t n = std::max<int64_t>(1, std::min({want, cap, (span + min_keys - 1) / min_keys}));
+  if (rows <= 64 || n < 8) return n;
+  return groups * (n / 8 * 8) >= 256 ? n / 8 * 8 : (n + 7) / 8 * 8;
 }
 
 // Shared body of dgg_attn_splitkv and of dgg_attn_decode / dgg_attn_decode_noalloc for grouped query heads (declared
@@ -399,6 +403,9 @@ int splitkv_launch(const char* op, const void* q, const void* k, const void* v, 
   sp.part_o = static_cast<float*>(workspace);
   sp.part_ml = sp.part_o + B * Hq * Sq * splits * D;
   sp.splits = (int)((span + chunk - 1) / chunk);  // slices that hold a key
+  // More than 64 rows: kept a multiple of 8 (splitkv_useful_splits) by slices without a key, which write empty partials
+  // (128 rows, 32 heads, 4,099 keys, 16 slices: 15 with a key 46.6 us, 16 41.3).
+  if (M > 64 && splits % 8 == 0) sp.splits = (sp.splits + 7) / 8 * 8;
   hipStream_t st = dgg::as_stream(stream);
   if (dtype == DGG_BF16) {
     if (D == 64) pick_splitkv<BF16, 64>(sp, nw, st);

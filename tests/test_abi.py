@@ -270,6 +270,15 @@ def test_clock_probe_validation(lib):
     assert lib.dgg_clock_probe(FAKE, 2_000_000, None) == E_SHAPE
 
 
+def test_split_counts_beyond_64_rows_are_multiples_of_8():
+    # several workgroups of rows share each key slice there, and only a multiple of 8 slices puts them on one XCD
+    from deepgengraph_amd.attention import splitkv_splits
+
+    for Sq, Hkv in ((64, 8), (128, 32), (20, 8), (33, 16)):
+        for span in [*range(2048, 6000, 131), 16383, 16384, 40001]:
+            assert splitkv_splits(1, Sq, 32, Hkv, span) % 8 == 0, (Sq, Hkv, span)
+
+
 def test_python_wrappers_reject_cpu_tensors():
     import torch
 
