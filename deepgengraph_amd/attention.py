@@ -473,9 +473,6 @@ def nonzero(x: torch.Tensor) -> torch.Tensor:
     return coords[: int(total.item())]
 
 
-TOPK_TWO_STAGE_N = 14336
-
-
 def topk_indices(scores: torch.Tensor, k: int, largest: bool = True) -> torch.Tensor:
     """deepgengraph_exp/cases/models/h2o.py:51-52 (torch.topk then sort of the indices) with a defined tie
     order: the k largest (largest=False: smallest, models/roco.py:55) of each row of scores [..., n] (fp32), ties
@@ -487,20 +484,16 @@ def topk_indices(scores: torch.Tensor, k: int, largest: bool = True) -> torch.Te
     n = scores.shape[-1]
     rows = scores.numel() // n if n else 0
     out = torch.empty(*scores.shape[:-1], k, dtype=torch.int64, device=scores.device)
-    # Rows of up to 65536 keys need no scratch memory; from TOPK_TWO_STAGE_N keys the library splits a row over several
-    # workgroups if it gets some (as much as a row just beyond 65536 keys needs).
-    ws = _select_workspace(rows, max(n, 65537) if n >= TOPK_TWO_STAGE_N and rows <= 64 else n, scores.device)
-    _lib.call("dgg_topk_select_ws", _lib.ptr(scores), rows, n, int(k), 1 if largest else 0, _lib.ptr(out),
-              _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.stream_handle(dev))
+    k = int(k)
+    ws = _scratch(_lib.load().dgg_topk_workspace_bytes(rows, n, k), scores.device)
+    _lib.call("dgg_topk", _lib.ptr(scores), rows, n, k, 1 if largest else 0, _lib.ptr(out), _lib.ptr(ws),
+              0 if ws is None else ws.numel(), _lib.stream_handle(dev))
     return out
 
 
-def _select_workspace(rows: int, n: int, device) -> torch.Tensor | None:
-    """Scratch of the selections over rows of more than 65536 keys (several workgroups per row); None below."""
-    need = int(_lib.load().dgg_select_workspace_bytes(rows, n))
-    if need <= 0:
-        return None
-    return torch.empty(need, dtype=torch.uint8, device=device)
+def _scratch(need: int, device) -> torch.Tensor | None:
+    """Scratch of the selections that run several workgroups per row; None where they need none."""
+    return torch.empty(need, dtype=torch.uint8, device=device) if need > 0 else None
 
 
 def roco_select(score: torch.Tensor, sq_score: torch.Tensor, q_len: int, recent: int, budget: int) -> torch.Tensor:
@@ -517,7 +510,7 @@ def roco_select(score: torch.Tensor, sq_score: torch.Tensor, q_len: int, recent:
     n = score.shape[-1]
     rows = score.numel() // n if n else 0
     out = torch.empty(*score.shape[:-1], budget + recent, dtype=torch.int64, device=score.device)
-    ws = _select_workspace(rows, n, score.device)
+    ws = _scratch(_lib.load().dgg_select_workspace_bytes(rows, n), score.device)
     _lib.call("dgg_roco_select_ws", _lib.ptr(score), _lib.ptr(sq_score), rows, n, int(q_len), int(recent),
               int(budget), _lib.ptr(out), _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.stream_handle(dev))
     return out

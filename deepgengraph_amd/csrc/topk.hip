@@ -1060,7 +1060,7 @@ int sel_check_ws(const char* op, int64_t rows, int64_t n, void* workspace, int64
   DGG_REQUIRE(rows < 65536, DGG_ERR_SHAPE, "%s: more than 65535 rows of over 65536 keys (got %lld rows)", op,
               (long long)rows);
   const int64_t need = sel_layout(rows, n, workspace, ws);
-  DGG_REQUIRE(workspace != nullptr, DGG_ERR_NULL, "%s: rows of more than 65536 keys need a workspace", op);
+  DGG_REQUIRE(workspace != nullptr, DGG_ERR_NULL, "%s: rows of this many keys need a workspace", op);
   DGG_REQUIRE(workspace_bytes >= need, DGG_ERR_WORKSPACE, "%s: workspace of %lld bytes < required %lld", op,
               (long long)workspace_bytes, (long long)need);
   DGG_REQUIRE(((uintptr_t)workspace & 255u) == 0, DGG_ERR_ALIGN, "%s: workspace must be 256-byte aligned", op);
@@ -1128,19 +1128,7 @@ extern "C" int64_t dgg_select_workspace_bytes(int64_t rows, int64_t n) {
 
 extern "C" int dgg_topk_select_ws(const float* scores, int64_t rows, int64_t n, int64_t k, int largest,
                                   int64_t* out_idx, void* workspace, int64_t workspace_bytes, void* stream) {
-  if (n <= 65536) {
-    // Where the caller has scratch memory and the rows alone do not fill the chip, the two-stage form spreads a row over
-    // a workgroup per 8,192 keys (kSel2MinN). Without scratch memory, or with many rows or a large k: one per row.
-    const bool two = n >= kSel2MinN && k >= 1 && k <= 2048 && rows >= 1 && rows <= 64 && scores && out_idx &&
-                     workspace != nullptr && ((uintptr_t)workspace & 255u) == 0 &&
-                     workspace_bytes >= sel_layout(rows, n, nullptr, nullptr);
-    if (!two) return dgg_topk_select(scores, rows, n, k, largest, out_idx, stream);
-    SelWs ws;
-    sel_layout(rows, n, workspace, &ws);
-    sel2_run(KeyScores{scores, (int)n, largest ? 1 : 0}, (int)rows, (int)n, (int)k, ws, kSelAll, out_idx, k,
-             dgg::as_stream(stream));
-    return dgg::check_launch("topk_indices");
-  }
+  if (n <= 65536) return dgg_topk_select(scores, rows, n, k, largest, out_idx, stream);
   DGG_REQUIRE(n <= kSelMaxN, DGG_ERR_SHAPE, "topk_indices: n must be <= 2^26 (got %lld)", (long long)n);
   DGG_REQUIRE(rows >= 0, DGG_ERR_SHAPE, "topk_indices: bad row count %lld", (long long)rows);
   DGG_REQUIRE(k >= 1 && k <= n, DGG_ERR_SHAPE, "topk_indices: k must be in [1, n] (got k=%lld, n=%lld)",
@@ -1160,6 +1148,30 @@ extern "C" int dgg_topk_select_ws(const float* scores, int64_t rows, int64_t n, 
   sel_run(kf, (int)rows, (int)n, ws, 0, (uint32_t)k, kSelAll, st);
   hipLaunchKernelGGL(sel_emit_kernel, dim3(ws.chunks, (unsigned)rows), dim3(kSelThreads), 0, st, (int)n, ws, 0, -1,
                      out_idx, (int)k);
+  return dgg::check_launch("topk_indices");
+}
+
+namespace {
+// Rows of at most 65,536 keys that take the two-stage form: spread over a workgroup per 8,192 keys where the rows alone do
+// not fill the chip (kSel2MinN has the measurements). With many rows or a large k: one workgroup per row.
+bool topk_two_stages(int64_t rows, int64_t n, int64_t k) {
+  return n >= kSel2MinN && n <= 65536 && k >= 1 && k <= 2048 && rows >= 1 && rows <= 64;
+}
+}  // namespace
+
+extern "C" int64_t dgg_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k) {
+  return topk_two_stages(rows, n, k) ? sel_layout(rows, n, nullptr, nullptr) : dgg_select_workspace_bytes(rows, n);
+}
+
+extern "C" int dgg_topk(const float* scores, int64_t rows, int64_t n, int64_t k, int largest, int64_t* out_idx,
+                        void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!topk_two_stages(rows, n, k))
+    return dgg_topk_select_ws(scores, rows, n, k, largest, out_idx, workspace, workspace_bytes, stream);
+  DGG_REQUIRE(scores && out_idx, DGG_ERR_NULL, "topk_indices: null pointer");
+  SelWs ws;
+  if (int rc = sel_check_ws("topk_indices", rows, n, workspace, workspace_bytes, &ws)) return rc;
+  sel2_run(KeyScores{scores, (int)n, largest ? 1 : 0}, (int)rows, (int)n, (int)k, ws, kSelAll, out_idx, k,
+           dgg::as_stream(stream));
   return dgg::check_launch("topk_indices");
 }
 

@@ -242,8 +242,7 @@ int dgg_roco_select(const float* score, const float* sq_score, int64_t rows, int
  * merge, reading the row once; others in radix passes; RoCo's `other` from the boundary of a two-stage `recent`,
  * in two reads of the row) through a caller-provided workspace of
  * dgg_select_workspace_bytes(rows, n) bytes (0 for n <= 65536, where these calls are dgg_topk_select /
- * dgg_roco_select and need none; a top-k given dgg_select_workspace_bytes(rows, 65537) bytes all the same runs in two
- * stages where that is faster), 256-byte aligned; rows <= 65535 when n > 65536. No counterpart in the
+ * dgg_roco_select and ignore the workspace), 256-byte aligned; rows <= 65535 when n > 65536. No counterpart in the
  * reference beyond the torch.topk calls they replace (models/h2o.py:51, models/snapkv.py:51, models/kf.py:54,
  * models/roco.py:54-61), which have no size limit. */
 int64_t dgg_select_workspace_bytes(int64_t rows, int64_t n);
@@ -252,6 +251,13 @@ int dgg_topk_select_ws(const float* scores, int64_t rows, int64_t n, int64_t k, 
 int dgg_roco_select_ws(const float* score, const float* sq_score, int64_t rows, int64_t n, int64_t q_len,
                        int64_t recent, int64_t budget, int64_t* out_idx, void* workspace, int64_t workspace_bytes,
                        void* stream);
+
+/* Top-k of rows of any length up to 2^26 in the fastest form: the results of dgg_topk_select, which it is for short rows;
+ * long rows, and those of up to 65536 keys that are few enough for it to pay, run over several workgroups each through a
+ * workspace of dgg_topk_workspace_bytes(rows, n, k) bytes (0: none is needed), 256-byte aligned. */
+int64_t dgg_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k);
+int dgg_topk(const float* scores, int64_t rows, int64_t n, int64_t k, int largest, int64_t* out_idx, void* workspace,
+             int64_t workspace_bytes, void* stream);
 
 /* Decode attention (Attn.forward with q_len == 1, attn.py:22-23: no mask) as split-KV + LSE merge.
  * q [B, Hq, D] strides {b,h}; k/v cache [B, Hkv, L, D] strides {b,h,l}; o [B, Hq, D] strides {b,h}.

@@ -223,6 +223,25 @@ def test_select_workspace_validation(lib):
     assert lib.dgg_roco_select_ws(None, None, 4, 1 << 20, 10, 0, 0, None, None, 0, None) == OK  # nothing to select
 
 
+def test_topk_any_length_validation(lib):
+    # two stages (scratch needed): 14336 to 65536 keys in at most 64 rows, k up to 2048; longer rows: as topk_select_ws
+    need = lib.dgg_topk_workspace_bytes(4, 20000, 100)
+    assert need > 0
+    for rows, n, k in ((4, 14335, 100), (65, 20000, 100), (4, 20000, 2049), (4, 20000, 0), (0, 20000, 10)):
+        assert lib.dgg_topk_workspace_bytes(rows, n, k) == 0
+    assert lib.dgg_topk_workspace_bytes(100, 1 << 20, 7) == lib.dgg_select_workspace_bytes(100, 1 << 20)
+    assert lib.dgg_topk_workspace_bytes(-1, 1 << 20, 7) == -1
+    ws = ctypes.c_void_p(0x100000)
+    assert lib.dgg_topk(FAKE, 4, 20000, 100, 1, FAKE, ws, need - 1, None) == E_WS
+    assert lib.dgg_topk(FAKE, 4, 20000, 100, 1, FAKE, None, need, None) == E_NULL
+    assert lib.dgg_topk(FAKE, 4, 20000, 100, 1, FAKE, ctypes.c_void_p(0x100010), need, None) == E_ALIGN
+    assert lib.dgg_topk(None, 4, 20000, 100, 1, FAKE, ws, need, None) == E_NULL
+    assert lib.dgg_topk(FAKE, 4, 20000, 20001, 1, FAKE, None, 0, None) == E_SHAPE
+    assert lib.dgg_topk(FAKE, 4, 100, 0, 1, FAKE, None, 0, None) == E_SHAPE
+    assert lib.dgg_topk(FAKE, 4, 1 << 20, 10, 1, FAKE, ws, 0, None) == E_WS
+    assert lib.dgg_topk(None, 0, 20000, 10, 1, None, None, 0, None) == OK
+
+
 def test_decode_noalloc_validation(lib):
     # every argument is checked before the device's scratch is looked up (no GPU needed for these)
     s = _strides([32 * 128, 128, 32 * 4096 * 128, 4096 * 128, 128] + [32 * 4096 * 128, 4096 * 128, 128] + [32 * 128, 128])

@@ -357,3 +357,17 @@ def test_topk_two_stages_by_choice(gpu, n, largest):
         assert lib.dgg_topk_select(_lib.ptr(x), 5, n, k, int(largest), _lib.ptr(want), _lib.stream_handle(gpu)) == 0
         got = A.topk_indices(x, k, largest=largest)
         assert torch.equal(got, want), f"n {n} k {k} largest {largest}"
+
+
+@pytest.mark.parametrize("n", [16384, 65536])
+def test_topk_select_ws_leaves_the_workspace_of_short_rows_alone(gpu, n):
+    """dgg_topk_select_ws ignores its workspace for rows of up to 65,536 keys (a caller may have it in use elsewhere),
+    whatever its size; the result is dgg_topk_select's."""
+    lib = _lib.load()
+    x = torch.randn(3, n, generator=torch.Generator(device=gpu).manual_seed(n), device=gpu)
+    ws = torch.full((lib.dgg_select_workspace_bytes(3, 1 << 17),), 0xA5, dtype=torch.uint8, device=gpu)
+    got, want = (torch.empty(3, 100, dtype=torch.int64, device=gpu) for _ in range(2))
+    stream = _lib.stream_handle(gpu)
+    assert lib.dgg_topk_select(_lib.ptr(x), 3, n, 100, 1, _lib.ptr(want), stream) == 0
+    assert lib.dgg_topk_select_ws(_lib.ptr(x), 3, n, 100, 1, _lib.ptr(got), _lib.ptr(ws), ws.numel(), stream) == 0
+    assert torch.equal(got, want) and bool((ws == 0xA5).all())
