@@ -82,8 +82,8 @@ def splitkv_splits(B: int, Sq: int, Hq: int, Hkv: int, span: int) -> int:
     """Key slices for a split-KV call over `span` keys: up to 512 workgroups (1024 for at most 8 rows per KV head, whose
     partials are small, and for more than 64, whose slices are long), each slice at least 32 keys and 8 per row it
     serves, and at most 64 slices below 16K keys, whose merge would take longer than the keys. Beyond 64 rows per KV head
-    a multiple of 8. The library's own rule for grouped-query decode (splitkv_useful_splits in csrc/splitkv.hip, with the
-    measurements)."""
+    a multiple of 8. dgg_attn_splitkv_splits without the call, whose conversions take longer than the sums;
+    splitkv_useful_splits in csrc/splitkv.hip has the measurements."""
     rows = (Hq // Hkv) * Sq
     groups = max(1, B * Hkv * (-(-rows // (32 if rows <= 32 else 64))))
     if rows > 64:  # several row groups read a slice: a multiple of 8 slices keeps them on one XCD and its L2
@@ -114,6 +114,8 @@ def decode_splits(B: int, Hq: int, L: int) -> int:
     16, 32, 8192                  2: 316  4: 315  16: 328  64: 362                   2
     2, 8, 65536                   4: 230  16: 93  32: 90  64: 96                    32
     ============================  ==============================================  ======
+
+    (dgg_attn_decode_splits without the call.)
     """
     want = max(-(-512 // max(1, B * Hq)), min(8, -(-L // 4096)))
     return int(max(1, min(1024, want, -(-L // 128))))
@@ -238,14 +240,19 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool
     return (out, lse) if return_lse else out
 
 
+def _splitkv_ws_floats(B: int, Sq: int, Hq: int, D: int, splits: int) -> int:
+    """dgg_attn_splitkv_workspace_bytes in floats, without the call (a microsecond of a decode step): an unnormalised
+    output row, its maximum and its sum per row and slice."""
+    return B * Sq * Hq * splits * (D + 2)
+
+
 def _splitkv(q, k, v, out, lse, causal, softcap, window, scale, lse_base2, splits, dev):
     B, Sq, Hq, D = q.shape
     Sk, Hkv = k.shape[1], k.shape[2]
     if splits is None:
         first = max(0, Sk - Sq - window + 1) if window else 0
         splits = splitkv_splits(B, Sq, Hq, Hkv, Sk - first)
-    # dgg_attn_splitkv_workspace_bytes: an unnormalised output row, its maximum and its sum per row and slice
-    ws = torch.empty(max(B * Sq * Hq * splits * (D + 2), 4), dtype=torch.float32, device=dev)
+    ws = torch.empty(max(_splitkv_ws_floats(B, Sq, Hq, D, splits), 4), dtype=torch.float32, device=dev)
     flags = (_lib.ATTN_CAUSAL if causal else 0) | (_lib.ATTN_LSE_BASE2 if lse_base2 else 0)
     strides = _strides3(q, k, v, out)
     _lib.call("dgg_attn_splitkv", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), _lib.ptr(lse), _lib.ptr(ws),

@@ -197,10 +197,11 @@ __global__ void __launch_bounds__(256) decode_merge_kernel(DecodeParams p) {
 // Splits a call runs with, of the `splits` it was given (its workspace is sized for those): enough for ~512 workgroups,
 // or up to 8 of at least 4,096 keys, and at least 128 keys each (one unrolled block of the partial kernel; with fewer
 // the block re-reads its last key). More splits only add partials and their merge. Measured on MI355X, D=128, bf16, at 64
-// splits and at the number this picks: B=64, H=32, L=128 855 -> 28 us (1); L=2048 895 -> 314 (1); B=16, L=1024 238 -> 45
+// splits and at the number this picks (attention.py's decode_splits has more shapes): B=64, H=32, L=128 855 -> 28 us (1); L=2048 895 -> 314 (1); B=16, L=1024 238 -> 45
 // (1); B=1, L=4096 35.8 -> 18.5 (16); B=64, L=8192 1445 -> 1229 (2).
 int64_t decode_useful_splits(int64_t splits, int64_t BH, int64_t L) {
-  const int64_t want = std::max((512 + BH - 1) / BH, std::min<int64_t>(8, (L + 4095) / 4096));
+  const int64_t want = std::max((511 + std::max<int64_t>(BH, 1)) / std::max<int64_t>(BH, 1),
+                                std::min<int64_t>(8, (L + 4095) / 4096));
   return std::max<int64_t>(1, std::min({splits, want, (L + 127) / 128}));
 }
 
@@ -216,6 +217,11 @@ void launch_decode(const DecodeParams& p, hipStream_t st) {
 extern "C" int64_t dgg_attn_decode_workspace_bytes(int64_t B, int64_t Hq, int64_t D, int64_t splits) {
   if (B < 0 || Hq < 0 || D < 0 || splits < 0) return -1;
   return B * Hq * splits * (D + 2) * (int64_t)sizeof(float);
+}
+
+extern "C" int64_t dgg_attn_decode_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t splits) {
+  if (B < 0 || Hq <= 0 || Hkv <= 0 || L < 1 || splits < 1) return -1;
+  return Hq > Hkv ? std::min(splits, dgg::splitkv_useful_splits(B, 1, Hq, Hkv, L)) : decode_useful_splits(splits, B * Hq, L);
 }
 
 namespace dgg {
@@ -257,7 +263,7 @@ int decode_launch(const char* op, const void* q, const void* k, const void* v, v
     // strides {b, l, h}; the partials have the same size.
     const int64_t st12[12] = {strides[0], 0,          strides[1], strides[2], strides[4], strides[3],
                               strides[5], strides[7], strides[6], strides[8], 0,          strides[9]};
-    splits = std::min(splits, dgg::splitkv_useful_splits(B, 1, Hq, Hkv, L));
+    splits = dgg_attn_decode_splits(B, Hq, Hkv, L, splits);
     return dgg::splitkv_launch(op, q, k, v, o, lse, workspace, workspace_bytes, B, 1, L, Hq, Hkv, D, st12, splits,
                                scale, 0.f, 0, 0u, dtype, stream, resolve_ws);
   }
@@ -284,7 +290,7 @@ int decode_launch(const char* op, const void* q, const void* k, const void* v, v
   p.Hkv = (int)Hkv;
   p.group = (int)(Hq / Hkv);
   p.L = (int)L;
-  splits = decode_useful_splits(splits, B * Hq, L);
+  splits = dgg_attn_decode_splits(B, Hq, Hkv, L, splits);
   p.chunk = (int)((L + splits - 1) / splits);
   p.splits = (int)((L + p.chunk - 1) / p.chunk);
   p.c = scale * kLog2e;

@@ -323,7 +323,7 @@ void pick_splitkv(const SplitParams& sp, int nw, hipStream_t st) {
 
 namespace dgg {
 
-// (attention.py's splitkv_splits is the same rule, for calls that size their own workspace.)
+// (dgg_attn_splitkv_splits hands it to callers, which size their own workspace; attention.py's splitkv_splits repeats it.)
 // A workgroup serves up to 32 rows of a KV head with one wave, 64 with two; a slice's latency is one tile of 32 keys after
 // another, so small calls want many short slices, as long as the partials (rows * (D + 2) floats a slice) stay small
 // against the keys and the merge short. Measured on MI355X, D=128, bf16, us at the number picked (and at a half and twice):
@@ -424,6 +424,11 @@ int splitkv_launch(const char* op, const void* q, const void* k, const void* v, 
 extern "C" int64_t dgg_attn_splitkv_workspace_bytes(int64_t B, int64_t Sq, int64_t Hq, int64_t D, int64_t splits) {
   if (B < 0 || Sq < 0 || Hq < 0 || D < 0 || splits < 0) return -1;
   return B * Hq * Sq * splits * (D + 2) * (int64_t)sizeof(float);
+}
+
+extern "C" int64_t dgg_attn_splitkv_splits(int64_t B, int64_t Sq, int64_t Hq, int64_t Hkv, int64_t span) {
+  if (B < 0 || Sq < 0 || Hq <= 0 || Hkv <= 0 || span < 0) return -1;
+  return dgg::splitkv_useful_splits(B, Sq, Hq, Hkv, span);
 }
 
 extern "C" int dgg_attn_splitkv(const void* q, const void* k, const void* v, void* o, float* lse, void* workspace,

@@ -267,6 +267,9 @@ int dgg_topk(const float* scores, int64_t rows, int64_t n, int64_t k, int larges
  * lse (optional): fp32 [B, Hq], natural log. splits in [1, 1024]: the most splits the call runs with (it takes fewer
  * where more would only add partials); L >= 1. */
 int64_t dgg_attn_decode_workspace_bytes(int64_t B, int64_t Hq, int64_t D, int64_t splits);
+/* The splits such a call runs with when given `splits` (an L that they do not divide may leave some without a key, which
+ * are left out). -1: a bad size. */
+int64_t dgg_attn_decode_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t splits);
 int dgg_attn_decode(const void* q, const void* k, const void* v, void* o, float* lse, void* workspace,
                     int64_t workspace_bytes, int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t D,
                     const int64_t* strides, int64_t splits, float scale, int dtype, void* stream);
@@ -281,6 +284,8 @@ int dgg_attn_decode(const void* q, const void* k, const void* v, void* o, float*
  * Sq >= 1, Sk >= 1, splits in [1, 1024]. dgg_attn_decode and dgg_attn_decode_noalloc run grouped-query calls
  * (Hq > Hkv) through these kernels with the same workspace size. */
 int64_t dgg_attn_splitkv_workspace_bytes(int64_t B, int64_t Sq, int64_t Hq, int64_t D, int64_t splits);
+/* The slice count that suits a call over `span` keys (those any of its rows sees). -1: a bad size. */
+int64_t dgg_attn_splitkv_splits(int64_t B, int64_t Sq, int64_t Hq, int64_t Hkv, int64_t span);
 int dgg_attn_splitkv(const void* q, const void* k, const void* v, void* o, float* lse, void* workspace,
                      int64_t workspace_bytes, int64_t B, int64_t Sq, int64_t Sk, int64_t Hq, int64_t Hkv, int64_t D,
                      const int64_t* strides, int64_t splits, float scale, float softcap, int64_t window,

@@ -289,6 +289,30 @@ def test_clock_probe_validation(lib):
     assert lib.dgg_clock_probe(FAKE, 2_000_000, None) == E_SHAPE
 
 
+def test_split_counts_and_workspace_are_the_librarys(lib):
+    # attention.py repeats three of the library's sums, to save the calls: equal over the sizes they are used at
+    import random
+
+    from deepgengraph_amd import attention as A
+
+    r = random.Random(0)
+    for _ in range(20000):
+        B, Hkv, G, Sq = r.choice([0, 1, 2, 7, 64]), r.choice([1, 2, 8, 32]), r.choice([1, 4, 7, 128]), r.randint(1, 300)
+        L, splits, D = int(2 ** r.uniform(0, 20)), r.randint(1, 1024), r.choice([64, 128, 256])
+        at = (B, Sq, Hkv * G, Hkv, L)
+        assert A.splitkv_splits(*at) == lib.dgg_attn_splitkv_splits(*at), at
+        assert A.decode_splits(B, Hkv, L) == lib.dgg_attn_decode_splits(B, Hkv, Hkv, L, 1024), at
+        assert 4 * A._splitkv_ws_floats(B, Sq, Hkv * G, D, splits) == lib.dgg_attn_splitkv_workspace_bytes(
+            B, Sq, Hkv * G, D, splits), at
+    # decode: the number given is the most; enough for 512 workgroups, or up to 8 of 4,096 keys, at least 128 keys each
+    for B, H, L, splits, runs in ((64, 32, 32768, 64, 8), (64, 32, 2048, 64, 1), (1, 32, 4096, 64, 16), (1, 32, 4096, 3, 3),
+                                  (1, 2, 33000, 1024, 256), (1, 2, 5, 16, 1), (2, 8, 65536, 1000, 32)):
+        assert lib.dgg_attn_decode_splits(B, H, H, L, splits) == runs
+    assert lib.dgg_attn_decode_splits(1, 32, 8, 4001, 64) == A.splitkv_splits(1, 1, 32, 8, 4001) == 64
+    assert lib.dgg_attn_decode_splits(0, 32, 32, 100, 64) == 1 and lib.dgg_attn_decode_splits(1, 32, 0, 100, 64) == -1
+    assert lib.dgg_attn_splitkv_splits(0, 4, 8, 8, 100) == 4 and lib.dgg_attn_splitkv_splits(1, 4, 8, 0, 100) == -1
+
+
 def test_split_counts_beyond_64_rows_are_multiples_of_8():
     # several workgroups of rows share each key slice there, and only a multiple of 8 slices puts them on one XCD
     from deepgengraph_amd.attention import splitkv_splits
