@@ -340,8 +340,12 @@ int64_t splitkv_useful_splits(int64_t B, int64_t Sq, int64_t Hq, int64_t Hkv, in
   // slices 207-222 us, 10 285, 11 321; 384 rows, 32 / 8 heads: 16 slices 104, 21 155). A span short of whole multiples
   // rounds down to one, or up where that leaves less than a workgroup per CU (256 rows, 32 / 8 heads: 2,100 keys 9
   // slices 23.8, 8 20.3; 3,000 keys 12 25.1, 8 22.3; 80 rows: 3,000 keys 12 17.0, 8 18.3, 16 15.9).
-  const int64_t want = rows > 64 ? std::max<int64_t>(8, 1024 / groups / 8 * 8)
-                                 : ((rows <= 8 ? 1024 : 512) + groups - 1) / groups;
+  // At most 8 rows: up to 960 workgroups, less than four per CU, so that no CU gets a fifth while the others wait (12 x 32 /
+  // 8 heads: 2,800 keys 11 slices, 1,056 workgroups, 36.6 us, 10 29.4; 32,768 keys 267, 244; 8 x 32,768 keys 16 slices 177,
+  // 15 169); with fewer than 16 groups 1,024 (32,768 keys 128 slices 29.3, 120 30.0).
+  int64_t want = ((rows <= 8 ? 1024 : 512) + groups - 1) / groups;
+  if (rows <= 8 && groups >= 16) want = 960 / groups >= 2 ? 960 / groups : (960 + groups - 1) / groups;
+  if (rows > 64) want = std::max<int64_t>(8, 1024 / groups / 8 * 8);
   const int64_t min_keys = std::max<int64_t>(32, 8 * std::min<int64_t>(rows, 32));
   const int64_t cap = span < 16384 ? 64 : 1024;
   const int64_t n = std::max<int64_t>(1, std::min({want, cap, (span + min_keys - 1) / min_keys}));

@@ -322,6 +322,15 @@ def test_split_counts_beyond_64_rows_are_multiples_of_8():
             assert splitkv_splits(1, Sq, 32, Hkv, span) % 8 == 0, (Sq, Hkv, span)
 
 
+def test_decode_steps_stay_within_four_workgroups_per_cu():
+    # one row per query head: a launch a little over 4 x 256 workgroups would end with a fifth round on a few CUs
+    from deepgengraph_amd.attention import splitkv_splits
+
+    for B in range(1, 61):
+        for span in (700, 3001, 9000, 32768):
+            assert 8 * B * splitkv_splits(B, 1, 32, 8, span) <= 1024, (B, span)
+
+
 def test_python_wrappers_reject_cpu_tensors():
     import torch
 
