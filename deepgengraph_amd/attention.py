@@ -79,8 +79,8 @@ def _splitkv_wide(B: int, Sq: int, Sk: int, Hq: int, D: int, window, ref_roundin
 
 
 def splitkv_splits(B: int, Sq: int, Hq: int, Hkv: int, span: int) -> int:
-    """Key slices for a split-KV call over `span` keys: up to 512 workgroups (960 to 1024 for at most 8 rows per KV head,
-    whose partials are small, and 1024 for more than 64, whose slices are long), each slice at least 32 keys and 8 per row it
+    """Key slices for a split-KV call over `span` keys: up to 512 workgroups (960 to 1024 for at most 8 rows per KV head and
+    768 for at most 16, whose partials are small, 1024 for more than 64, whose slices are long), each slice at least 32 keys and 8 per row it
     serves, and at most 64 slices below 16K keys, whose merge would take longer than the keys. Beyond 64 rows per KV head
     a multiple of 8. dgg_attn_splitkv_splits without the call, whose conversions take longer than the sums;
     splitkv_useful_splits in csrc/splitkv.hip has the measurements."""
@@ -88,10 +88,15 @@ def splitkv_splits(B: int, Sq: int, Hq: int, Hkv: int, span: int) -> int:
     groups = max(1, B * Hkv * (-(-rows // (32 if rows <= 32 else 64))))
     if rows > 64:  # several row groups read a slice: a multiple of 8 slices keeps them on one XCD and its L2
         want = max(8, 1024 // groups // 8 * 8)
-    elif rows <= 8 and groups >= 16:  # fewer than four workgroups per CU, so that none gets a fifth
-        want = 960 // groups if groups <= 480 else -(-960 // groups)
     else:
-        want = -(-(1024 if rows <= 8 else 512) // groups)
+        target = 512
+        if rows <= 8:
+            target = 960 if groups >= 16 else 1024
+        elif rows <= 16 and (groups < 32 or span < 24576):
+            target = 768
+        want = target // groups if target in (960, 768) else 0  # whole workgroups per CU
+        if want < 2:
+            want = -(-target // groups)
     min_keys = max(32, 8 * min(rows, 32))
     n = int(max(1, min(want, 64 if span < 16384 else 1024, -(-span // min_keys))))
     if rows <= 64 or n < 8:

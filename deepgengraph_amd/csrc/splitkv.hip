@@ -326,7 +326,7 @@ namespace dgg {
 // (dgg_attn_splitkv_splits hands it to callers, which size their own workspace; attention.py's splitkv_splits repeats it.)
 // A workgroup serves up to 32 rows of a KV head with one wave, 64 with two; a slice's latency is one tile of 32 keys after
 // another, so small calls want many short slices, as long as the partials (rows * (D + 2) floats a slice) stay small
-// against the keys and the merge short. Measured on MI355X, D=128, bf16, us at the number picked (and at a half and twice):
+// against the keys and the merge short. Measured on MI355X, D=128, bf16, us at some number of slices (and at others):
 // B=1, 1 row, 32 / 8 heads: 4,001 keys 64: 9.7 (32: 10.8, 8: 22.2); 1,024 keys 32: 7.8 (16: 9.0); 32,768 keys 128: 27.2
 // (64: 29.5, 256: 28.6). B=8, 4,001 keys 16: 28.2 (8: 29.4, 32: 29.7). 16 rows, 32 heads: 8,192 keys 16: 30.8 (8: 39.8,
 // 32: 31.3); 2,048 keys 16: 14.3 (8: 15.9, 32: 16.4). 16 rows, 32 / 8 heads: 8,192 keys 32: 19.1 (16: 23.2, 64: 21.9).
@@ -343,8 +343,12 @@ int64_t splitkv_useful_splits(int64_t B, int64_t Sq, int64_t Hq, int64_t Hkv, in
   // At most 8 rows: up to 960 workgroups, less than four per CU, so that no CU gets a fifth while the others wait (12 x 32 /
   // 8 heads: 2,800 keys 11 slices, 1,056 workgroups, 36.6 us, 10 29.4; 32,768 keys 267, 244; 8 x 32,768 keys 16 slices 177,
   // 15 169); with fewer than 16 groups 1,024 (32,768 keys 128 slices 29.3, 120 30.0).
-  int64_t want = ((rows <= 8 ? 1024 : 512) + groups - 1) / groups;
-  if (rows <= 8 && groups >= 16) want = 960 / groups >= 2 ? 960 / groups : (960 + groups - 1) / groups;
+  // 9 to 16 rows: up to 768, but 512 from 32 groups and 24K keys, as for more rows (16 rows: 2 x 32 / 8 heads, 28,000
+  // keys 32 slices 49.2, 48 45.0; 2 x 32 heads, 7,500 keys 8 51.2, 12 47.4, but 32,768 keys 170, 180, one of them 16 92.9, 24
+  // 94.6; 64 rows, 32 / 8 heads, 32,768 keys 64 36.3, 96 39.4).
+  const int64_t target = rows <= 8 ? (groups >= 16 ? 960 : 1024) : rows <= 16 && (groups < 32 || span < 24576) ? 768 : 512;
+  int64_t want = target == 960 || target == 768 ? target / groups : 0;
+  if (want < 2) want = (target + groups - 1) / groups;
   if (rows > 64) want = std::max<int64_t>(8, 1024 / groups / 8 * 8);
   const int64_t min_keys = std::max<int64_t>(32, 8 * std::min<int64_t>(rows, 32));
   const int64_t cap = span < 16384 ? 64 : 1024;

@@ -322,13 +322,16 @@ def test_split_counts_beyond_64_rows_are_multiples_of_8():
             assert splitkv_splits(1, Sq, 32, Hkv, span) % 8 == 0, (Sq, Hkv, span)
 
 
-def test_decode_steps_stay_within_four_workgroups_per_cu():
+def test_split_counts_fill_the_chip_evenly():
     # one row per query head: a launch a little over 4 x 256 workgroups would end with a fifth round on a few CUs
     from deepgengraph_amd.attention import splitkv_splits
 
     for B in range(1, 61):
         for span in (700, 3001, 9000, 32768):
             assert 8 * B * splitkv_splits(B, 1, 32, 8, span) <= 1024, (B, span)
+    # 9 to 16 rows: three per CU (two were slower than the rule before them had been at 28,000 and 7,500 keys)
+    assert splitkv_splits(2, 4, 32, 8, 28000) == 48 and splitkv_splits(2, 16, 32, 32, 7500) == 12
+    assert splitkv_splits(2, 16, 32, 32, 32768) == 8 and splitkv_splits(1, 16, 32, 32, 32768) == 16
 
 
 def test_python_wrappers_reject_cpu_tensors():
