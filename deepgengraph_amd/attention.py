@@ -64,18 +64,28 @@ def _splitkv_shaped(Sq: int, Sk: int, Hq: int, Hkv: int, ref_rounding: bool, dty
             and not ref_rounding and dtype in (torch.float16, torch.bfloat16))
 
 
-# Longer query blocks go there too (head_dim 128) while the prefill kernel has at most one 64-row workgroup per CU, so
-# that its time is the serial chain of the keys: up to SPLITKV_WIDE_QLEN query rows, over at least 32 keys per query row
-# (40 beyond 128 rows). Measured on MI355X, bf16, B=1, prefill / split-KV, us: 64 rows 32 / 8 heads 2,048 keys 22.0 / 19.4,
-# 8,192 68 / 36, 32,768 255 / 72; 128 rows 32 heads 4,096 keys 42.7 / 37.6, 32,768 441 / 149, but 2,048 keys 24.1 / 28.8;
-# 256 rows 32 / 8 heads 32,768 keys 260 / 218, but 8,192 keys 71 / 75; 384 rows: never.
+# Longer query blocks go there too (head_dim 128) while the prefill kernel leaves most of the chip idle, so that its time is
+# the serial chain of the keys: up to SPLITKV_WIDE_QLEN query rows, over at least 32 keys per query row (40 beyond 128 rows), and
+# with at most 128 groups of 64 rows that share a KV head. The split kernels do the same products in every group, so
+# their time grows with the groups, the chain's only with the keys: at least 32 keys per group, 64 with grouped query heads (whose
+# keys and values, being fewer, the prefill kernel finds in the caches). Measured on MI355X, bf16, prefill / split-KV, us,
+# keys and values not in the caches: B=1, 100 rows, 32 heads, 4,100 keys (64 groups) 39.6 / 38.6, 128 rows, 32,768 keys 441 /
+# 149; B=2, 100 rows, 32 heads, 4,100 (128) 62.5 / 56.5; B=4, 100 rows, 32 heads, 4,100 (256) 70.0 / 111.6; 32 / 8 heads: B=1,
+# 128 rows, 4,224 (64) 36.1 / 36.0, B=1, 65 rows, 2,165 (40) 22.0 / 23.9, B=2, 100 rows, 4,100 (112) 37.4 / 45.8, B=4, 64
+# rows, 2,164 (128) 23.3 / 40.1.
 SPLITKV_WIDE_QLEN = 256
 
 
-def _splitkv_wide(B: int, Sq: int, Sk: int, Hq: int, D: int, window, ref_rounding: bool, dtype) -> bool:
+def _splitkv_wide(B: int, Sq: int, Sk: int, Hq: int, D: int, window, ref_rounding: bool, dtype,
+                  Hkv: int | None = None) -> bool:
+    if not (D == 128 and 1 <= Sq <= SPLITKV_WIDE_QLEN and not ref_rounding
+            and dtype in (torch.float16, torch.bfloat16)):
+        return False
+    Hkv = Hkv or Hq
     span = min(Sk, window + Sq - 1) if window else Sk
-    return (D == 128 and 1 <= Sq <= SPLITKV_WIDE_QLEN and span >= max((32 if Sq <= 128 else 40) * Sq, SPLITKV_MIN_KEYS)
-            and B * Hq * (-(-Sq // 64)) <= 256 and not ref_rounding and dtype in (torch.float16, torch.bfloat16))
+    groups = B * Hkv * (-(-(Hq // Hkv) * Sq // 64))
+    return (span >= max((32 if Sq <= 128 else 40) * Sq, SPLITKV_MIN_KEYS, (32 if Hq == Hkv else 64) * groups)
+            and groups <= 128)
 
 
 def splitkv_splits(B: int, Sq: int, Hq: int, Hkv: int, span: int) -> int:
@@ -235,7 +245,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool
             lse.copy_(lse1.view(B, Hq, 1) * (math.log2(math.e) if lse_base2 else 1.0))
         return (out, lse) if return_lse else out
     if (_splitkv_shaped(Sq, Sk, Hq, Hkv, ref_rounding, q.dtype)
-            or _splitkv_wide(B, Sq, Sk, Hq, D, window, ref_rounding, q.dtype)):
+            or _splitkv_wide(B, Sq, Sk, Hq, D, window, ref_rounding, q.dtype, Hkv)):
         _splitkv(q, k, v, out, lse, causal, softcap, window, scale, lse_base2, None, dev)
         return (out, lse) if return_lse else out
     flags = ((_lib.ATTN_CAUSAL if causal else 0) | (_lib.ATTN_REF_ROUNDING if ref_rounding else 0)

@@ -334,6 +334,21 @@ def test_split_counts_fill_the_chip_evenly():
     assert splitkv_splits(2, 16, 32, 32, 32768) == 8 and splitkv_splits(1, 16, 32, 32, 32768) == 16
 
 
+def test_wide_query_blocks_leave_the_prefill_kernel_what_it_does_faster():
+    # batches of query blocks whose 64-row groups fill the chip (the split kernels took 1.2 to 2 times as long)
+    import torch
+
+    from deepgengraph_amd.attention import _splitkv_wide
+
+    def wide(B, Sq, Sk, Hq, Hkv):
+        return _splitkv_wide(B, Sq, Sk, Hq, 128, 0, False, torch.bfloat16, Hkv)
+
+    assert not wide(4, 100, 4100, 32, 32) and not wide(4, 100, 4100, 32, 8) and not wide(2, 100, 4100, 32, 8)
+    assert not wide(4, 64, 2164, 32, 8) and not wide(1, 65, 2165, 32, 8)
+    assert wide(1, 100, 4100, 32, 32) and wide(2, 100, 4100, 32, 32) and wide(1, 128, 4224, 32, 8)
+    assert wide(1, 256, 32768, 32, 8) and not wide(2, 256, 32768, 32, 8) and not wide(2, 100, 4095, 32, 32)
+
+
 def test_python_wrappers_reject_cpu_tensors():
     import torch
 
