@@ -224,11 +224,13 @@ def test_select_workspace_validation(lib):
 
 
 def test_topk_any_length_validation(lib):
-    # two stages (scratch needed): 14336 to 65536 keys in at most 64 rows, k up to 2048; longer rows: as topk_select_ws
+    # two stages (scratch needed): 16384 (15361 for k > 512) to 65536 keys in at most 64 rows, k up to 2048; longer rows: as
+    # topk_select_ws
     need = lib.dgg_topk_workspace_bytes(4, 20000, 100)
     assert need > 0
-    for rows, n, k in ((4, 14335, 100), (65, 20000, 100), (4, 20000, 2049), (4, 20000, 0), (0, 20000, 10)):
+    for rows, n, k in ((4, 16383, 512), (4, 15360, 513), (65, 20000, 100), (4, 20000, 2049), (4, 20000, 0), (0, 20000, 10)):
         assert lib.dgg_topk_workspace_bytes(rows, n, k) == 0
+    assert lib.dgg_topk_workspace_bytes(4, 16384, 512) > 0 and lib.dgg_topk_workspace_bytes(4, 15361, 513) > 0
     assert lib.dgg_topk_workspace_bytes(100, 1 << 20, 7) == lib.dgg_select_workspace_bytes(100, 1 << 20)
     assert lib.dgg_topk_workspace_bytes(-1, 1 << 20, 7) == -1
     ws = ctypes.c_void_p(0x100000)

@@ -339,7 +339,7 @@ def test_column_forms_agree(gpu, S, dtype):
 
 
 @pytest.mark.parametrize("largest", [True, False])
-@pytest.mark.parametrize("n", [14335, 14336, 16385, 40000, 65536])
+@pytest.mark.parametrize("n", [14335, 14336, 15360, 15361, 16383, 16384, 16385, 40000, 65536])
 def test_topk_two_stages_by_choice(gpu, n, largest):
     """Rows around and above the length from which topk_indices splits a row over several workgroups, against the
     one-workgroup form: exact, with ties across the chunks, NaN and infinities, k at the limits of the prefilter."""
