@@ -354,9 +354,11 @@ constexpr int kSelNSel = 3;                                 // selections a work
 // with the 64-per-lane merge; 32 keys per lane spill 124 VGPRs and 164 SGPRs).
 constexpr int kSel2Per = 8;                                 // keys per lane in the first stage
 constexpr int kSel2Chunk = 64 * kSel2Per * kTopkWaves;      // keys per workgroup
-// Shortest row that takes the two-stage form by choice. Top-256 of 32 rows, one workgroup per row / two stages, us: 12,288
-// keys 17.2 / 17.7, 16,384 23.0 / 17.0, 32,768 50.8 / 18.1, 65,536 81.9 / 19.0.
-constexpr int kSel2MinN = 14336;
+// Shortest row that takes the two-stage form by choice: the one-workgroup form is faster below (its threads' segments reach
+// 16 keys beyond 15,360, all on one LDS bank group), with the prefilter up to 16,383 keys. One workgroup per row / two stages,
+// 32 rows, us: top-256 of 14,336 keys 16.1 / 19.0, 15,872 20.4 / 21.0, 16,384 20.6 / 19.1, 16,385 38.2 / 19.2, 65,536 82 / 19;
+// top-1,000 of 14,336 19.7 / 21.0, 15,000 20.4 / 21.0, 15,872 24.2 / 21.0.
+constexpr int sel2_min_n(int64_t k) { return k <= kTopkThreads / 2 ? 16384 : 15361; }
 constexpr int kSel2MaxCand = 64 * kTopkThreads;             // candidates per row
 constexpr int kSel2C2 = 16384;  // second-level candidates per row (groups * k <= 65,536 / 8 + k, see sel2_run)
 
@@ -1153,9 +1155,9 @@ extern "C" int dgg_topk_select_ws(const float* scores, int64_t rows, int64_t n, 
 
 namespace {
 // Rows of at most 65,536 keys that take the two-stage form: spread over a workgroup per 8,192 keys where the rows alone do
-// not fill the chip (kSel2MinN has the measurements). With many rows or a large k: one workgroup per row.
+// not fill the chip (sel2_min_n has the measurements). With many rows or a large k: one workgroup per row.
 bool topk_two_stages(int64_t rows, int64_t n, int64_t k) {
-  return n >= kSel2MinN && n <= 65536 && k >= 1 && k <= 2048 && rows >= 1 && rows <= 64;
+  return n >= sel2_min_n(k) && n <= 65536 && k >= 1 && k <= 2048 && rows >= 1 && rows <= 64;
 }
 }  // namespace
 
