@@ -143,7 +143,8 @@ __device__ void radix_kstar(const uint32_t (&key)[PER], uint64_t cand, uint32_t 
 // lanes on a few hot bins; after this a few lanes per instruction are left. One barrier pair, against ~5 for a pass.
 // For k up to half a lane maximum per thread (beyond, little drops out) and at least 8 keys per lane (top-256 of 32 rows:
 // 1,048,576 keys 142.5 -> 121.6 us, 131,072 25.7 -> 24.4; at 4 keys per lane it costs more than it saves, 2,048 keys
-// 7.3 -> 8.1). Every thread calls this with the same k.
+// 7.3 -> 8.1). Every thread calls this with the same k. A wave with fewer than ceil(k / 16) lanes that hold a candidate makes
+// T 0, and the work is for nothing: see prefilter_pays.
 template <int PER>
 __device__ uint64_t radix_prefilter(const uint32_t (&key)[PER], uint64_t cand, uint32_t k, TopkShared& sh) {
   if (PER < 8 || k > kTopkThreads / 2) return cand;
@@ -167,12 +168,21 @@ __device__ uint64_t radix_prefilter(const uint32_t (&key)[PER], uint64_t cand, u
   return cand;
 }
 
+// Whether the prefilter helps a selection of k from n keys dealt out by segment(): from 6 keys a thread, if the segments reach
+// far enough into the last wave (ceil(n / 1024) keys each, the first threads first). Without this line top-256 of 64 rows
+// took, us, without / with the prefilter: 4,097 keys (5 a thread, 820 threads) 12.3 / 14.0, 6,800 14.4 / 15.9, 16,385 (964
+// threads) 35.3 / 38.7; with enough threads 6,000 13.4 / 13.0, 8,192 17.6 / 16.4, 16,384 24.6 / 20.5.
+__device__ __forceinline__ bool prefilter_pays(int n, int k) {
+  const int per = (n + kTopkThreads - 1) / kTopkThreads, threads = (n + per - 1) / per;
+  return per >= 6 && threads >= kTopkThreads - 64 + max(8, (k + kTopkWaves - 1) / kTopkWaves);
+}
+
 template <int PER>
-__device__ uint64_t radix_take(const uint32_t (&key)[PER], uint64_t cand, uint32_t k, TopkShared& sh,
+__device__ uint64_t radix_take(const uint32_t (&key)[PER], uint64_t cand, uint32_t k, TopkShared& sh, bool prefilter,
                                uint32_t* bound = nullptr) {
   if (k == 0) return 0;
   uint32_t prefix, remaining;
-  cand = radix_prefilter<PER>(key, cand, k, sh);
+  if (prefilter) cand = radix_prefilter<PER>(key, cand, k, sh);
   radix_kstar<PER>(key, cand, k, sh, prefix, remaining, bound != nullptr);
   if (bound != nullptr && threadIdx.x == 0) {  // K* and how many keys equal to it are taken
     bound[0] = prefix;
@@ -246,7 +256,7 @@ __global__ void __launch_bounds__(kTopkThreads) topk_kernel(const float* __restr
     key[j] = j < cnt ? order_key(x[seg0 + j]) : 0u;
     if (!largest) key[j] = ~key[j];  // the smallest first; NaN (all ones) becomes the least
   }
-  const uint64_t take = radix_take<PER>(key, all, (uint32_t)k, sh);
+  const uint64_t take = radix_take<PER>(key, all, (uint32_t)k, sh, prefilter_pays(n, k));
   write_taken(take, 0, seg0, out + (int64_t)blockIdx.x * k, (uint32_t)k, sh);
 }
 
@@ -307,7 +317,11 @@ __global__ void __launch_bounds__(kTopkThreads) roco_select_kernel(const float* 
   }
 #pragma unroll
   for (int j = 0; j < PER; ++j) key[j] = j < cnt ? order_key(roco_mean(s1[row + seg0 + j], rcp)) : 0u;
-  const uint64_t pick = radix_take<PER>(key, other, (uint32_t)budget, sh);    // roco.py:57-58
+  // Beyond 16 keys a thread the masks leave no registers for the prefilter, and it pays later: 64 rows, recent / budget, us,
+  // without / with: 17,000 keys 64 / 64 94.9 / 98.4, 32,768 163.9 / 155.5; 256 / 256 28,000 137 / 142, 40,000 186 / 182;
+  // 0 / 512 40,000 135 / 142, 50,000 195 / 193.
+  const bool pf = prefilter_pays(n, budget) && (PER <= 16 || n >= 24576 + 48 * budget);
+  const uint64_t pick = radix_take<PER>(key, other, (uint32_t)budget, sh, pf);  // roco.py:57-58
   write_taken(pick, rec, seg0, out + (int64_t)blockIdx.x * (budget + recent), (uint32_t)(budget + recent), sh);
 }
 
@@ -856,7 +870,8 @@ sel2_local_kernel(KeyF kf, int n, int k, SelWs ws, int cand_sel) {
   }
   if (kk == 0) return;  // (uniform over the workgroup)
   uint32_t kstar, rem;
-  valid = radix_prefilter<kSel2Per>(key, valid, kk, sh);
+  // (a row's last chunk, if not whole, leaves waves without a key: see prefilter_pays)
+  if (n - c0 >= kSel2Chunk) valid = radix_prefilter<kSel2Per>(key, valid, kk, sh);
   radix_kstar<kSel2Per>(key, valid, kk, sh, kstar, rem, false);
   // ranks of the keys equal to K* in index order (wave, step, lane), then the taken keys' slots in the same order
   const uint64_t lt = (1ull << lane) - 1;
@@ -917,7 +932,7 @@ __global__ void __launch_bounds__(kTopkThreads) sel2_merge_kernel(SelWs ws, cons
 #pragma unroll
   for (int j = 0; j < PER; ++j) key[j] = j < cnt ? kp[seg0 + j] : 0u;
   const uint64_t take =
-      radix_take<PER>(key, all, (uint32_t)k, sh, bound ? sel_bound(ws, blockIdx.x) : nullptr);
+      radix_take<PER>(key, all, (uint32_t)k, sh, prefilter_pays(m, k), bound ? sel_bound(ws, blockIdx.x) : nullptr);
   write_taken_gather(take, seg0, ip, out + (int64_t)blockIdx.x * out_rs, (uint32_t)k, sh);
 }
 
@@ -939,7 +954,7 @@ __global__ void __launch_bounds__(kTopkThreads) sel2_group_kernel(SelWs ws, int 
   uint32_t key[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) key[j] = j < cnt ? kp[seg0 + j] : 0u;
-  uint64_t take = radix_take<PER>(key, all, (uint32_t)k, sh);
+  uint64_t take = radix_take<PER>(key, all, (uint32_t)k, sh, prefilter_pays(cnt_g, k));
   uint32_t tot;
   uint32_t pos = block_exclusive_scan(__popcll(take), sh.wsum, tot);
   uint32_t* ok = ws.c2key + row * kSel2C2 + (int64_t)blockIdx.x * k;

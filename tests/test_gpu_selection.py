@@ -371,3 +371,21 @@ def test_topk_select_ws_leaves_the_workspace_of_short_rows_alone(gpu, n):
     assert lib.dgg_topk_select(_lib.ptr(x), 3, n, 100, 1, _lib.ptr(want), stream) == 0
     assert lib.dgg_topk_select_ws(_lib.ptr(x), 3, n, 100, 1, _lib.ptr(got), _lib.ptr(ws), ws.numel(), stream) == 0
     assert torch.equal(got, want) and bool((ws == 0xA5).all())
+
+
+@pytest.mark.parametrize("n,k", [(5120, 256), (6144, 512), (7736, 64), (7744, 64), (7928, 512), (7936, 512), (16385, 256),
+                                 (17000, 16), (27647, 64), (27648, 64), (40000, 512)])
+def test_selection_around_the_prefilters_line(gpu, n, k):
+    """Rows and counts on either side of the lines from which the one-workgroup selections run the prefilter (threads with
+    keys in the last wave; keys per thread; RoCo's own line beyond 16): exact, with ties, against the oracle."""
+    g = torch.Generator().manual_seed(n + k)
+    x = torch.stack([torch.randn(n, generator=g), torch.randint(0, 50, (n,), generator=g).float()])
+    lib = _lib.load()
+    xg, got = x.to(gpu), torch.empty(2, k, dtype=torch.int64, device=gpu)
+    assert lib.dgg_topk_select(_lib.ptr(xg), 2, n, k, 1, _lib.ptr(got), _lib.stream_handle(gpu)) == 0
+    np.testing.assert_array_equal(got.cpu().numpy(), osel.topk_indices(x.numpy(), k))
+    s1 = torch.rand(2, n, generator=g) * 100
+    s1[1] = torch.randint(1, 60, (n,), generator=g).float()
+    s2 = s1 * s1 / n + torch.rand(2, n, generator=g)
+    rec = A.roco_select(s1.to(gpu), s2.to(gpu), n, 64, k).cpu().numpy()
+    np.testing.assert_array_equal(rec, osel.roco_select(s1.numpy(), s2.numpy(), n, 64, k))
