@@ -163,6 +163,13 @@ def bench_prefill(args, dev):
                 clock_mhz=[_clock_mhz(clk, 0), _clock_mhz(clk, 1)], steady=steady)
 
 
+def _decode_splits(B, Hq, Hkv, L, splits):
+    """The splits a decode call runs with when given `splits`."""
+    from deepgengraph_amd import _lib
+
+    return _lib.load().dgg_attn_decode_splits(B, Hq, Hkv, L, splits)
+
+
 def bench_decode(args, dev):
     from deepgengraph_amd import attention as A
     from deepgengraph_amd import configs as C
@@ -178,7 +185,7 @@ def bench_decode(args, dev):
     torch.cuda.empty_cache()
     gbps = nbytes / (ms * 1e-3) / 1e9
     res = dict(workload=cfg.name, ms=round(ms, 4), bytes=nbytes, gbps=round(gbps, 1),
-               frac=round(gbps / PEAK_HBM_GBPS, 4), splits=cfg.splits)
+               frac=round(gbps / PEAK_HBM_GBPS, 4), splits=_decode_splits(cfg.B, cfg.Hq, cfg.Hkv, cfg.L, cfg.splits))
     # The same decode through the drop-in compile(Attn) callable: q [B, 1, H, D] and the cache in the case layout
     # [B, L, H, D] (attn.py:18-34 with q_len == 1), routed to the split-KV kernels by attention().
     from deepgengraph_amd import cases as tcases
@@ -331,14 +338,15 @@ def bench_splitkv(args, dev):
     q = torch.randn(B, Hq, D, generator=g, device=dev).half()
     kc = torch.randn(B, Hkv, L, D, generator=g, device=dev).half()
     vc = torch.randn(B, Hkv, L, D, generator=g, device=dev).half()
-    splits = 8  # best of 8 .. 128 in a sweep on MI355X (6.13 vs 5.80 TB/s at 64)
+    splits = 8  # the most; the call runs with as many as suit it
     ws = torch.empty(A.decode_workspace_bytes(B, Hq, D, splits), dtype=torch.uint8, device=dev)
     out = torch.empty_like(q)
     ms, info = _variant(lambda: A.decode_attention(q, kc, vc, splits=splits, out=out, workspace=ws), 10)
     nb = 2 * (2 * kc.numel() + 2 * q.numel())
     gbps = nb / (ms * 1e-3) / 1e9
     res[f"gqa_decode_b{B}_h{Hq}/{Hkv}_kv{L}_d{D}_f16"] = dict(ms=round(ms, 4), gbps=round(gbps, 1),
-                                                             frac=round(gbps / PEAK_HBM_GBPS, 4), splits=splits,
+                                                             frac=round(gbps / PEAK_HBM_GBPS, 4),
+                                                             splits=_decode_splits(B, Hq, Hkv, L, splits),
                                                              **info)
     del q, kc, vc, ws, out
     torch.cuda.empty_cache()

@@ -548,9 +548,9 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                      scale: float | None = None, return_lse: bool = False, out: torch.Tensor | None = None,
                      workspace: torch.Tensor | None = None):
     """Attn.forward with q_len == 1 (attn.py:22-23: nothing masked) over a [B, Hkv, L, D] KV cache, computed as a
-    split-KV pass (`splits` slices of the cache) followed by a log-sum-exp merge. q [B, Hq, D] -> out
-    [B, Hq, D] (+ lse [B, Hq] fp32). `workspace` (uint8/any, >= decode_workspace_bytes bytes) may be passed to
-    avoid an allocation per call."""
+    split-KV pass followed by a log-sum-exp merge. `splits`: the most slices the cache is cut into (it takes fewer
+    where more would only add partials). q [B, Hq, D] -> out [B, Hq, D] (+ lse [B, Hq] fp32). `workspace` (uint8/any,
+    >= decode_workspace_bytes bytes) may be passed to avoid an allocation per call."""
     dev = _lib.require_gpu(q, k_cache, v_cache, out, workspace)
     if q.dim() != 3 or k_cache.dim() != 4 or v_cache.shape != k_cache.shape:
         raise RuntimeError("decode_attention: expected q [B, Hq, D] and k/v caches [B, Hkv, L, D]")
