@@ -389,3 +389,46 @@ def test_selection_around_the_prefilters_line(gpu, n, k):
     s2 = s1 * s1 / n + torch.rand(2, n, generator=g)
     rec = A.roco_select(s1.to(gpu), s2.to(gpu), n, 64, k).cpu().numpy()
     np.testing.assert_array_equal(rec, osel.roco_select(s1.numpy(), s2.numpy(), n, 64, k))
+
+
+@pytest.mark.parametrize("D,Sq,Sk,Hq,Hkv,causal,window,dtype,row_pad", [
+    (128, 200, 512, 4, 4, 1, 0, torch.float16, 0),      # Sq < Sk
+    (128, 300, 164, 4, 4, 1, 0, torch.bfloat16, 0),     # Sq > Sk: 136 rows see no key; 36 keys in the last tile
+    (128, 640, 640, 4, 4, 1, 70, torch.float16, 0),     # a window that starts past tile 0, tiles in rotated order
+    (128, 260, 700, 4, 4, 0, 90, torch.bfloat16, 0),    # a window without a causal mask
+    (128, 130, 260, 8, 2, 0, 0, torch.float16, 0),      # no mask, grouped heads, 4 keys in the last tile
+    (128, 129, 96, 4, 1, 1, 0, torch.bfloat16, 12),     # 32 keys in the last tile, exp_rand rows longer than the keys
+    (128, 33, 4, 2, 2, 1, 0, torch.float16, 0),         # one chunk of keys
+    (128, 200, 333, 4, 2, 1, 0, torch.float16, 3),      # keys and rows off 16 bytes (the register-staged kernel)
+    (128, 130, 200, 1, 1, 1, 0, torch.float16, 4100000),  # exp_rand rows too far apart for 32-bit lane offsets
+    (64, 200, 512, 4, 2, 1, 100, torch.bfloat16, 0),
+])
+def test_keyformer_row_pass(gpu, D, Sq, Sk, Hq, Hkv, causal, window, dtype, row_pad):
+    """dgg_attn_kf_rowlse by itself, over what the entry point accepts beyond the KeyFormer case (kf.py:36-39 is causal with
+    Sq == Sk), against the log-sum-exp in 64 bits. fp32 scores: the sums of up to 700 terms and exponents of a size of 10 are
+    within 700 * 2^-24 + 10 * 2^-23 < 5e-5 of exact (base-2 logarithm)."""
+    B, tau = 2 if row_pad < 1000 else 1, 1.5
+    g = torch.Generator(device=gpu).manual_seed(Sq + Sk)
+    q = torch.randn(B, Sq, Hq, D, generator=g, device=gpu).to(dtype)
+    k = torch.randn(B, Sk, Hkv, D, generator=g, device=gpu).to(dtype)
+    rs = Sk + row_pad
+    er = torch.empty(B * Hq * Sq * rs, device=gpu).as_strided((B, Hq, Sq, Sk), (Hq * Sq * rs, Sq * rs, rs, 1))
+    er.copy_(1.0 + torch.randn(B, Hq, Sq, Sk, generator=g, device=gpu).abs())
+    lse2 = torch.full((B, Hq, Sq), float("nan"), device=gpu)
+    strides = _lib.int64_array([*q.stride()[:3], *k.stride()[:3]])
+    _lib.call("dgg_attn_kf_rowlse", _lib.ptr(q), _lib.ptr(k), _lib.ptr(er), _lib.int64_array(er.stride()[:3]),
+              _lib.ptr(lse2), B, Sq, Sk, Hq, Hkv, D, strides, D ** -0.5, tau, window, causal, _lib.dtype_code(dtype),
+              _lib.stream_handle(gpu))
+    qc, kc = q.double().cpu().transpose(1, 2), k.double().cpu().transpose(1, 2).repeat_interleave(Hq // Hkv, dim=1)
+    y = (torch.matmul(qc, kc.transpose(2, 3).contiguous()) * D ** -0.5 - er.double().cpu().log()) / tau
+    rel = torch.arange(Sq).unsqueeze(1) + (Sk - Sq) - torch.arange(Sk)
+    hidden = torch.zeros(Sq, Sk, dtype=torch.bool)
+    if causal:
+        hidden |= rel < 0
+    if window:
+        hidden |= rel >= window
+    ref = torch.logsumexp(y.masked_fill(hidden, float("-inf")), dim=-1) / np.log(2.0)
+    out = lse2.double().cpu()
+    assert torch.equal(torch.isinf(out), torch.isinf(ref)) and not torch.isnan(out).any()
+    fin = torch.isfinite(ref)
+    assert (out[fin] - ref[fin]).abs().max().item() < 5e-5
