@@ -605,8 +605,8 @@ __global__ void __launch_bounds__(kThreads) attn_colsum_kernel(AttnParams p) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Column-sum kernel for head_dim 128. A workgroup of NW waves owns 32*NW keys; wave w keeps keys
-// k0 + 32w .. + 31 in VGPRs as the B operand. Query tiles of BQ rows stream through an NSTAGE ring in LDS
+// Column-sum kernel for head_dim 128. A workgroup of NW waves owns 32*NW/NG keys, which each of its NG row groups
+// covers; a wave keeps 32 of them in VGPRs as the B operand. Query tiles of BQ rows stream through a two-stage ring in LDS
 // with the forward's swizzled layout and direct-to-LDS copies (the Q tile takes the place of the K tile),
 // each stage followed by the BQ lse values of its rows (global_load_lds_dword, issued by the last wave).
 // S (BQ x 32) = Q . K^T puts one key per lane: accumulator register j of block mb holds query row

@@ -231,11 +231,9 @@ __device__ __forceinline__ void map_block_kv_window(int n_tiles, int B, int Hq, 
 }
 
 // ------------------------------------------------------------------------------------------------
-// Forward kernel for head_dim 128 and 256 ("DMA kernel"). NW waves of 32*NQB query rows each; K/V tiles of BN
-// keys are copied global -> LDS by the direct-to-LDS loads of gfx950 (no VGPR staging, no LDS store
-// instructions) into an NSTAGE ring, with one barrier per tile. head_dim 128 runs 8 waves at two per SIMD;
-// head_dim 256 (Q 64 + O 128 VGPRs per lane) runs 4 waves at one per SIMD. Each 16-byte chunk c of tile row r
-// sits at
+// LDS layout of the tiles that direct-to-LDS loads of gfx950 bring in (no VGPR staging, no LDS store instructions): K / V in
+// the forwards, Q in the column passes, K in KeyFormer's row pass. For head_dim 128 and 256 each 16-byte chunk c of
+// tile row r sits at
 //     (r/4)*GROUP_B + (r%4)*ROW_B + 16*(c ^ 4*(r%4))        (ROW_B = 2*D bytes, 4-row groups padded by 16 bytes)
 // which keeps both the K fragment reads (16 lanes, 16 rows, one chunk) and the V transposing reads (4 rows x
 // 4 chunks per 16-lane group) on distinct LDS banks; the direct loads write that layout by fetching, for LDS
