@@ -90,9 +90,9 @@ def _splitkv_wide(B: int, Sq: int, Sk: int, Hq: int, D: int, window, ref_roundin
 
 def splitkv_splits(B: int, Sq: int, Hq: int, Hkv: int, span: int) -> int:
     """Key slices for a split-KV call over `span` keys: up to 512 workgroups (960 to 1024 for at most 8 rows per KV head and
-    768 for at most 16, whose partials are small, 1024 for more than 64, whose slices are long), each slice at least 32 keys and 8 per row it
-    serves, and at most 64 slices below 16K keys, whose merge would take longer than the keys. Beyond 64 rows per KV head
-    a multiple of 8. dgg_attn_splitkv_splits without the call, whose conversions take longer than the sums;
+    768 for at most 16, whose partials are small, 1024 for more than 64, whose slices are long), each slice at least 32
+    keys and 8 per row it serves, and at most 64 slices below 16K keys, whose merge would take longer than the keys.
+    Beyond 64 rows per KV head a multiple of 8. dgg_attn_splitkv_splits without the call, whose conversions take longer than the sums;
     splitkv_useful_splits in csrc/splitkv.hip has the measurements."""
     rows = (Hq // Hkv) * Sq
     groups = max(1, B * Hkv * (-(-rows // (32 if rows <= 32 else 64))))

@@ -197,8 +197,8 @@ __global__ void __launch_bounds__(256) decode_merge_kernel(DecodeParams p) {
 // Splits a call runs with, of the `splits` it was given (its workspace is sized for those): enough for ~512 workgroups,
 // or up to 8 of at least 4,096 keys, and at least 128 keys each (one unrolled block of the partial kernel; with fewer
 // the block re-reads its last key). More splits only add partials and their merge. Measured on MI355X, D=128, bf16, at 64
-// splits and at the number this picks (attention.py's decode_splits has more shapes): B=64, H=32, L=128 855 -> 28 us (1); L=2048 895 -> 314 (1); B=16, L=1024 238 -> 45
-// (1); B=1, L=4096 35.8 -> 18.5 (16); B=64, L=8192 1445 -> 1229 (2).
+// splits and at the number this picks (attention.py's decode_splits has more shapes): B=64, H=32, L=128 855 -> 28 us (1);
+// L=2048 895 -> 314 (1); B=16, L=1024 238 -> 45 (1); B=1, L=4096 35.8 -> 18.5 (16); B=64, L=8192 1445 -> 1229 (2).
 int64_t decode_useful_splits(int64_t splits, int64_t BH, int64_t L) {
   const int64_t want = std::max((511 + std::max<int64_t>(BH, 1)) / std::max<int64_t>(BH, 1),
                                 std::min<int64_t>(8, (L + 4095) / 4096));

@@ -327,8 +327,8 @@ __global__ void __launch_bounds__(kTopkThreads) roco_select_kernel(const float* 
 
 // ------------------------------------------------------------------------------------------------
 // Rows longer than 65536 keys (through dgg_topk from sel2_min_n(k), in two stages): the same selections (same key order,
-// same tie rule, same output order) over many workgroups per row, through a caller-provided workspace, in one of two forms. A selection of k with
-// ceil(n / kSel2Chunk) * k <= kSel2MaxCand runs in two stages (sel2_local_kernel, sel2_merge_kernel): each chunk's k
+// same tie rule, same output order) over many workgroups per row, through a caller-provided workspace, in one of two
+// forms. A selection of k with ceil(n / kSel2Chunk) * k <= kSel2MaxCand runs in two stages (sel2_local_kernel, sel2_merge_kernel): each chunk's k
 // largest as candidates, then k among those, reading the row once. Other selections run in passes: a row is cut into
 // chunks of kSelChunk keys, one 256-thread workgroup per (chunk, row); wave w of a chunk owns its contiguous
 // kSelWaveSpan keys, 64 at a time (lane l on key 64i + l), so a 64-bit ballot is one aligned word of a bit mask.
